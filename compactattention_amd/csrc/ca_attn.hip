@@ -11,9 +11,14 @@
 //  - The G query heads of a KV group share the group's block table, so a KV row
 //    (request, kv head) owns Lq*G "packed" query rows r = t*G + g (token t, head g).
 //  - A workgroup (8 waves, one per CU) takes 256 packed rows; each wave keeps 32 rows (one
-//    32x32 MFMA tile) for the whole KV loop: Q in VGPRs, O^T in accumulators.  Each SIMD
-//    runs two waves whose softmax and MFMA phases overlap; a wave raises its issue
-//    priority while it feeds the S^T MFMAs.
+//    32x32 MFMA tile) for the whole KV loop: Q in VGPRs, O^T in accumulators.
+//  - The loop is software-pipelined inside each wave: the scores of the next block run on the
+//    matrix cores beside the softmax of this one, then its PV product beside the next block's
+//    row max, instruction by instruction (fused below).  Bound: matrix-core issue and power.
+//    At 2048 queries over 32768 dense keys (32 Q / 8 KV heads) a 64-key step of a SIMD's two
+//    waves takes about 3000 cycles for 2176 of MFMA work (72 % busy) where it took 3700 (57 %),
+//    but the part lowers its clock as the matrix cores fill (1.75 -> 1.5 GHz), so the launch
+//    gains 6-7 % (966 -> 906 us); with the loop's LDS reads left out it would gain another 9 %.
 //  - Scores are computed transposed, S^T = K Q^T (A = K from LDS, B = Q from VGPRs), so the
 //    softmax output lands in exactly the VGPR layout the second product's B operand needs:
 //    O^T += V^T P^T (A = V^T from LDS).  Inside each 32-key S^T tile the A-row -> key map
@@ -23,9 +28,8 @@
 //    row-major with XOR swizzles that keep the fragment reads free of bank conflicts.  V^T
 //    fragments are read with the gfx950 transposing LDS read (ds_read_b64_tr_b16), two
 //    per MFMA.
-//  - Four LDS stages: the DMA of the next three blocks is in flight while the current
-//    block is computed, and a step waits only for the block after it.  Optional split of
-//    each row's block list (split-KV) with an LSE merge.
+//  - Rings of four K and four V blocks in LDS; the DMA runs two (V) and three (K) blocks ahead.
+//    Optional split of each row's block list (split-KV) with an LSE merge.
 //  - Workgroup ids are remapped so consecutive work items (same KV row) share an XCD and
 //    its L2.
 
@@ -39,6 +43,7 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef float f32x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
@@ -48,11 +53,11 @@ typedef __attribute__((address_space(3))) void lds_void_t;
 typedef __attribute__((address_space(3))) i16x4_t lds_i16x4_t;
 
 constexpr int kNW = 8;     // waves per workgroup (32 packed query rows each)
-constexpr int kStages = 4;  // LDS stages (K + V of one block each): 128 KB per workgroup
+constexpr int kStages = 4;  // places of the K and of the V ring in LDS: 128 KB per workgroup
 constexpr int kBM = 32 * kNW;        // packed query rows per workgroup
 constexpr int kKBytes = 64 * 256;  // K rows of one block in LDS (swizzled, unpadded)
 constexpr int kVBytes = 64 * 256;  // V rows of one block in LDS (swizzled, unpadded)
-constexpr int kStageBytes = kKBytes + kVBytes;
+constexpr int kVRing = kStages * kKBytes;  // LDS byte offset of the V ring
 constexpr float kRescale = 8.0f;      // lazy-rescale slack (log2 units)
 
 struct AttnParams {
@@ -76,11 +81,6 @@ struct AttnParams {
     // row's selected count is within 1.5x of their mean (workgroup 0 records the choice
     // here for the merge); null otherwise
     int32_t* ws_unsplit;
-    // K and V without page tables, 64-token blocks contiguous in token order (stride_blk =
-    // 64 stride_tok) and every request's tokens within 2^31 bytes: the DMA addresses a block
-    // through one buffer resource per KV row (the block's byte offset in the scalar offset),
-    // whose range ends at the request's last token as the per-block resources do
-    int row_res;
     int32_t qpos0[CA_MAX_BATCH];     // absolute position of each request's query row 0
     int32_t nkb[CA_MAX_BATCH];       // valid logical blocks of each request
     int32_t sp[CA_MAX_BATCH];        // splits of each request's block lists
@@ -120,6 +120,25 @@ typedef const __attribute__((address_space(4))) int32_t const_i32_t;
 __device__ __forceinline__ int32_t sload(const int32_t* p) {
     return *(const_i32_t*)p;
 }
+// Words of a raw buffer resource over `bytes` bytes at base (wave-uniform).
+__device__ __forceinline__ u32x4_t buffer_words(const uint16_t* base, int bytes) {
+    const uint64_t a = reinterpret_cast<uint64_t>(base);
+    return u32x4_t{static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(a))),
+                   static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(a >> 32) & 0xffff)),
+                   static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(bytes)), 0x00020000u};
+}
+// One LDS-DMA load: lane L's 16 bytes at byte offset off of the resource go to LDS byte dst + 16 L.
+__device__ __forceinline__ void dma_lds(u32x4_t rsrc, int off, uint32_t dst) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds"
+                 :
+                 : "v"(off), "s"(rsrc), "s"(dst)
+                 : "memory");
+}
+template <int N>
+struct IntC {
+    static constexpr int value = N;
+};
+#define CA_PIN() asm volatile("" ::: "memory")
 // Completes this wave's outstanding LDS-DMA loads (vector-memory counter).
 __device__ __forceinline__ void wait_dma() {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -132,10 +151,10 @@ __device__ __forceinline__ void wait_dma() {
 // CU (128 KB of LDS).
 // kTab: block lists come from the per-row table (prefill); otherwise they are the identity
 // 0 .. nkb-1 (dense decode).
-template <int NW, bool kTab>
+template <int NW, bool kTab, bool kRow>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) void attn_fwd_kernel(AttnParams p) {
     constexpr int BM = 32 * NW;
-    __shared__ __attribute__((aligned(16))) uint8_t smem[kStages * kStageBytes];  // [stage]: K rows, then V rows
+    __shared__ __attribute__((aligned(16))) uint8_t smem[kStages * (kKBytes + kVBytes)];  // K ring, then V ring
 
     // Ragged launches whose row tiles fill 3/4 of the CUs: one round of row tiles is enough
     // when the rows' selected counts are even, so the items of the other splits have nothing
@@ -290,7 +309,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
     const int32_t* kpt = p.k.page_table ? p.k.page_table + (int64_t)row * p.k.pts : nullptr;
     const int32_t* vpt = p.v.page_table ? p.v.page_table + (int64_t)row * p.v.pts : nullptr;
 
-    // ---- global -> LDS staging of one block (LDS DMA) ----
+    // ---- global -> LDS staging of one block's K or V rows (LDS DMA) ----
     // A block is 64 K rows and 64 V rows of 256 bytes.  Each wave issues 2 + 2 buffer loads
     // that write LDS directly (1 KB per instruction: lane L fills bytes 16L..16L+15 of the
     // instruction's 4 rows); the lane chooses which global 16-byte chunk lands there, which
@@ -299,7 +318,10 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
     //   K: 16-byte chunk c of row r sits at chunk c ^ (r & 15)    (conflict-free b128 reads)
     //   V: 16-byte chunk c of row r sits at chunk c ^ 4 (r & 3)   (conflict-free transposed reads)
     // 32-bit offsets inside a block (the host checks 64 * stride_tok < 2^30) on top of a
-    // wave-uniform block base in the buffer resource.
+    // wave-uniform block base in the buffer resource.  The loads are issued from inline asm
+    // (they have no register outputs): the compiler does not see the LDS writes, so it does
+    // not put vmcnt(0) in front of the LDS reads; the waits before the barriers below are
+    // counted by hand.
     static_assert(NW == 8, "the staging split assumes eight waves");
     const int wu = __builtin_amdgcn_readfirstlane(w);
     const int st_row = 4 * wu + (l >> 4);
@@ -313,42 +335,50 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
     // and 0 * V must not meet a non-finite V).  Row offsets go in the VGPR offset, which the
     // range check covers.
     const int kv_tokens = qpos0 + s.Lq;
-    const __amdgpu_buffer_rsrc_t rk_row =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(kbase_row), 0, kv_tokens * kstok_b, 0x00020000);
-    const __amdgpu_buffer_rsrc_t rv_row =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(vbase_row), 0, kv_tokens * vstok_b, 0x00020000);
-    const int kblk_b = 64 * kstok_b;
-    const int vblk_b = 64 * vstok_b;
-    auto issue_block = [&](int e, int stage) {
-        const int kb = block_id(e);
-        if (p.row_res) {
-            uint8_t* kdst = smem + stage * kStageBytes + wu * 1024;
-            uint8_t* vdst = kdst + kKBytes;
+    const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(to_lds(smem))) + wu * 1024;
+    // Where a block's rows are: its logical id (kRow: the offset in the row's one resource) and
+    // its K and V pages.  The id nkb, the block after the request's last, stands for no block:
+    // its loads are out of the buffer's range, touch no memory and write zeros.
+    struct Blk {
+        int id, kp, vp;
+    };
+    const u32x4_t k_rsrc = buffer_words(kbase_row, kRow ? kv_tokens * kstok_b : 0);
+    const u32x4_t v_rsrc = buffer_words(vbase_row, kRow ? kv_tokens * vstok_b : 0);
+    auto load_half = [&](const uint16_t* base_row, u32x4_t rsrc, int64_t sblk, int stok_b, int goff, int id, int page,
+                         int half, uint32_t dst) {
+        int off = goff + half * 32 * stok_b;
+        if (kRow)
             // the block offset goes in the vector offset, which the range check covers (the
             // scalar offset is not checked)
-            const int ko = k_goff + kb * kblk_b;
-            const int vo = v_goff + kb * vblk_b;
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(rk_row, to_lds(kdst + i * 8192), 16, ko + i * 32 * kstok_b, 0, 0, 0);
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(rv_row, to_lds(vdst + i * 8192), 16, vo + i * 32 * vstok_b, 0, 0, 0);
-            }
-            return;
+            off += id * 64 * stok_b;
+        else
+            rsrc = buffer_words(base_row + page * sblk, max(min(kv_tokens - id * 64, 64), 0) * stok_b);
+        dma_lds(rsrc, off, dst + half * 8192);
+    };
+    // The list's blocks, 64 entries at a time in registers (lane i: entry 64 c + i, no block past
+    // the list's end), so a step's block is a v_readlane and no load; the next 64 are loaded
+    // while these are used.
+    Blk next = {0, 0, 0}, cur = {0, 0, 0};
+    auto load_blks = [&](int c) {
+        const int e = e0 + 64 * c + l;
+        if (e >= e1) return Blk{nkb, 0, 0};
+        const int id = kTab ? min(max(tab[e], 0), nkb - 1) : e;
+        if (kRow) return Blk{id, 0, 0};
+        return Blk{id, kpt ? static_cast<int>(clamp_page(kpt[id], p.k.max_page)) : id,
+                   vpt ? static_cast<int>(clamp_page(vpt[id], p.v.max_page)) : id};
+    };
+    auto next_blk = [&](int i) {  // entry i, asked for in ascending order
+        if ((i & 63) == 0) {
+            cur = next;
+            next = load_blks((i >> 6) + 1);
         }
-        const int64_t kphys = kpt ? clamp_page(sload(kpt + kb), p.k.max_page) : kb;
-        const int64_t vphys = vpt ? clamp_page(sload(vpt + kb), p.v.max_page) : kb;
-        const int rows = min(kv_tokens - kb * 64, 64);
-        const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<uint16_t*>(kbase_row + kphys * p.k.sblk), 0, rows * kstok_b, 0x00020000);
-        const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<uint16_t*>(vbase_row + vphys * p.v.sblk), 0, rows * vstok_b, 0x00020000);
-        uint8_t* kdst = smem + stage * kStageBytes + wu * 1024;
-        uint8_t* vdst = kdst + kKBytes;
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, to_lds(kdst + i * 8192), 16, k_goff + i * 32 * kstok_b, 0, 0, 0);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, to_lds(vdst + i * 8192), 16, v_goff + i * 32 * vstok_b, 0, 0, 0);
+        const int u = i & 63;
+        Blk b = {__builtin_amdgcn_readlane(cur.id, u), 0, 0};
+        if (!kRow) {
+            b.kp = __builtin_amdgcn_readlane(cur.kp, u);
+            b.vp = __builtin_amdgcn_readlane(cur.vp, u);
         }
+        return b;
     };
 
     const float sl2 = p.scale_log2;
@@ -370,115 +400,250 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
     const int v_x = 2 * ((l >> 4) & 1) + ((l & 3) >> 1);
     int v_off[4];
 #pragma unroll
-    for (int dt = 0; dt < 4; ++dt) v_off[dt] = (8 * h + v_rq) * 256 + (4 * (dt ^ v_rq) + v_x) * 16 + (l & 1) * 8;
-    auto process = [&](int kb, const uint8_t* stage_base, bool masked) {
-        const uint8_t* ks = stage_base;
-        const uint8_t* vs = stage_base + kKBytes;
-        f32x16_t sacc[2];
+    for (int dt = 0; dt < 4; ++dt)
+        v_off[dt] = kVRing + (8 * h + v_rq) * 256 + (4 * (dt ^ v_rq) + v_x) * 16 + (l & 1) * 8;
+    // The normaliser sums the bf16-rounded weights the PV product uses: the 16-block 4x4x4 MFMA
+    // with a ones A operand adds each lane's own four values (its column of its block) to every
+    // element of the lane's accumulator.  (v_dot2 does the same in the VALU's encoding but waits
+    // for a running MFMA to end: the loop took 2.18M cycles with it where it takes 1.53M now.)
+    const i16x4_t ones = {0x3f80, 0x3f80, 0x3f80, 0x3f80};
+    auto add_weights = [&](uint32_t w0, uint32_t w1, f32x4_t acc) {
+        const u32x2_t w = {w0, w1};
+        return __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(ones, __builtin_bit_cast(i16x4_t, w), acc, 0, 0, 0);
+    };
+
+    f32x16_t sc[2];  // scores of the block whose softmax comes next (32 keys each)
+    float m_neg = 0.0f;  // -m_run of that block (0 while a row has seen no key)
+    auto k_frag = [&](int base, int i) {
+        return *reinterpret_cast<const bf16x8_t*>(smem + base + k_off[i >> 1] + (i & 1) * 8192);
+    };
+    auto v_frag = [&](int base, int i) {  // A operand of PV MFMA i: 16-key step i / 4, 32-d tile i % 4
+        const uint8_t* vp = smem + base + v_off[i & 3] + (i >> 2) * 4096;
+        const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(to_lds_v4(vp));
+        const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(to_lds_v4(vp + 1024));
+        return __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+    };
+    auto scores = [&](int kbase) {
 #pragma unroll
         for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-            for (int j = 0; j < 16; ++j) sacc[kt][j] = 0.0f;
-        // the two 32-key accumulators alternate so consecutive MFMAs are independent; the
-        // K fragment reads run six ahead of the MFMAs (scheduling groups below)
-        __builtin_amdgcn_s_setprio(1);
-        {
-            bf16x8_t kfr[16];
+            for (int j = 0; j < 16; ++j) sc[kt][j] = 0.0f;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) kfr[i] = *reinterpret_cast<const bf16x8_t*>(ks + k_off[i >> 1] + (i & 1) * 8192);
+        for (int i = 0; i < 16; ++i)
+            sc[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k_frag(kbase, i), qf[i >> 1], sc[i & 1], 0, 0, 0);
+    };
+    auto mask = [&](int kb) {
+        // value j of half kt holds key kt*32 + swap23(8*(j/4) + 4*h + j%4)
+        // = kt*32 + 8*h + key_off(j); visible iff kb*64 + key <= qpos0 + t
+        const int vis = qpos0 + qtok - kb * 64 - 8 * h;
 #pragma unroll
-            for (int i = 0; i < 16; ++i)
-                sacc[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kfr[i], qf[i >> 1], sacc[i & 1], 0, 0, 0);
-            __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);  // 6 LDS reads
+        for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-            for (int i = 0; i < 10; ++i) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // 1 MFMA
-                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // 1 LDS read
+            for (int j = 0; j < 16; ++j) {
+                const int key = kt * 32 + 16 * (j >> 3) + 4 * ((j >> 2) & 1) + (j & 3);
+                if (key > vis) sc[kt][j] = -__builtin_inff();
             }
-            __builtin_amdgcn_sched_group_barrier(0x008, 6, 0);
-        }
-        __builtin_amdgcn_s_setprio(0);
-        if (masked) {
-            // value j of half kt holds key kt*32 + swap23(8*(j/4) + 4*h + j%4)
-            // = kt*32 + 8*h + key_off(j); visible iff kb*64 + key <= qpos0 + t
-            const int vis = qpos0 + qtok - kb * 64 - 8 * h;
-#pragma unroll
-            for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-                for (int j = 0; j < 16; ++j) {
-                    const int key = kt * 32 + 16 * (j >> 3) + 4 * ((j >> 2) & 1) + (j & 3);
-                    if (key > vis) sacc[kt][j] = -__builtin_inff();
-                }
-        }
-        float mx = -__builtin_inff();
-#pragma unroll
-        for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-            for (int j = 0; j < 16; ++j) mx = fmaxf(mx, sacc[kt][j]);
-        mx = xor32_max(mx) * sl2;
+    };
+    // The running max of each row rises to mx (both lane halves' row max, scaled) where mx
+    // exceeds it by more than kRescale; the accumulators are rescaled.  Called when some lane
+    // of the wave needs it.
+    auto rise = [&](float mx) {
         float alpha = 1.0f;
         if (mx > m_run + kRescale) {
             alpha = __builtin_amdgcn_exp2f(m_run - mx);  // 0 when m_run = -inf
             m_run = mx;
+            m_neg = -mx;
             l_run *= alpha;
         }
-        if (__ballot(alpha != 1.0f)) {
 #pragma unroll
-            for (int dt = 0; dt < 4; ++dt)
+        for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
-                for (int j = 0; j < 16; ++j) oacc[dt][j] *= alpha;
-        }
-        const float m_use = m_run == -__builtin_inff() ? 0.0f : m_run;
+            for (int j = 0; j < 16; ++j) oacc[dt][j] *= alpha;
+    };
+    auto block_max = [&]() {
+        float mx = -__builtin_inff();
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+            for (int j = 0; j < 16; ++j) mx = fmaxf(mx, sc[kt][j]);
+        mx = xor32_max(mx) * sl2;
+        if (__ballot(mx > m_run + kRescale)) rise(mx);
+    };
+    // softmax of sc and O^T += V^T P^T
+    auto finish = [&](int vbase) {
         bf16x8_t pf[4];
-        float rs = 0.0f;
-        const bf16x2_t ones = {static_cast<__bf16>(1.0f), static_cast<__bf16>(1.0f)};
+        f32x4_t rs = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int s4 = 0; s4 < 4; ++s4) {
             f32x8_t pv8;
 #pragma unroll
             for (int i = 0; i < 8; ++i)
-                pv8[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[s4 >> 1][8 * (s4 & 1) + i], sl2, -m_use));
+                pv8[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[s4 >> 1][8 * (s4 & 1) + i], sl2, m_neg));
             pf[s4] = __builtin_convertvector(pv8, bf16x8_t);
-            // the normaliser sums the bf16-rounded weights the PV product uses
-            rs = __builtin_amdgcn_fdot2_f32_bf16(__builtin_shufflevector(pf[s4], pf[s4], 0, 1), ones, rs, false);
-            rs = __builtin_amdgcn_fdot2_f32_bf16(__builtin_shufflevector(pf[s4], pf[s4], 2, 3), ones, rs, false);
-            rs = __builtin_amdgcn_fdot2_f32_bf16(__builtin_shufflevector(pf[s4], pf[s4], 4, 5), ones, rs, false);
-            rs = __builtin_amdgcn_fdot2_f32_bf16(__builtin_shufflevector(pf[s4], pf[s4], 6, 7), ones, rs, false);
+            const u32x4_t w4 = __builtin_bit_cast(u32x4_t, pf[s4]);
+            rs = add_weights(w4[0], w4[1], rs);
+            rs = add_weights(w4[2], w4[3], rs);
         }
-        l_run += rs;  // this lane's half of the row; combined across lanes n, n+32 at the end
+        l_run += rs[0];  // this lane's half of the row; combined across lanes n, n+32 at the end
 #pragma unroll
-        for (int s4 = 0; s4 < 4; ++s4) {
-#pragma unroll
-            for (int dt = 0; dt < 4; ++dt) {
-                const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(to_lds_v4(vs + v_off[dt] + s4 * 4096));
-                const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(to_lds_v4(vs + v_off[dt] + s4 * 4096 + 1024));
-                const bf16x8_t a = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-                oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, pf[s4], oacc[dt], 0, 0, 0);
+        for (int i = 0; i < 16; ++i)
+            oacc[i & 3] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v_frag(vbase, i), pf[i >> 2], oacc[i & 3], 0, 0, 0);
+    };
+    // ---- KV loop ----
+    // Slot j computes the scores of block j + 1 (its first half) and the PV product of block j
+    // (its second half); the slots have one barrier each, between the halves.  The barrier of
+    // slot j stands for: K of block j + 2 and V of block j + 1 have landed, and every wave has
+    // read K of block j + 1 and V of block j - 1.  So slot j issues V of block j + 3 and K of
+    // block j + 5 after it, into the places of those two in rings of four blocks, and the
+    // loads stay in flight for two (V) and three (K) slots.  Every slot issues its four loads
+    // (blocks past the list's end load nothing), so the counts of the waits are constants.
+    const int nblk = e1 - e0;
+    Blk vq0, vq1;  // the two entries whose K is issued and V is not
+    auto issue_k = [&](int i, int half, const Blk& b) {
+        load_half(kbase_row, k_rsrc, p.k.sblk, kstok_b, k_goff, b.id, b.kp, half, lds0 + (i & 3) * 16384);
+    };
+    auto issue_v = [&](int i, int half, const Blk& b) {
+        load_half(vbase_row, v_rsrc, p.v.sblk, vstok_b, v_goff, b.id, b.vp, half, lds0 + kVRing + (i & 3) * 16384);
+    };
+    auto mid_slot = [&]() {
+        // K of j + 3, V of j + 2 and K of j + 4 may stay in flight
+        asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        CA_PIN();
+    };
+    auto issue_slot = [&](int j) {
+        const Blk nb = next_blk(j + 5);
+        for (int half = 0; half < 2; ++half) issue_v(j + 3, half, vq0);
+        for (int half = 0; half < 2; ++half) issue_k(j + 5, half, nb);
+        vq0 = vq1;
+        vq1 = nb;
+    };
+    // The pipelined slot: the scores of the next block (K in ring place R + 1) beside the
+    // softmax of sc, then its PV product (V in place R) beside the rest of the softmax and the
+    // next block's row max.  kf holds the first kAhead K fragments on entry and those of the
+    // next slot on return.  The pins fix the order of the instructions in groups of one MFMA, a
+    // fragment read and the stages of one weight: its fma, the exp2 of the weight before, the
+    // pack of the pair before that and the sum of the four before, so no instruction of a group
+    // waits for another.
+    constexpr int kAhead = 4;   // K fragments in flight ahead of their MFMA
+    constexpr int kVAhead = 3;  // V fragments
+    bf16x8_t kf[16];
+    auto fused = [&](f32x16_t(&sc)[2], f32x16_t(&sn)[2], auto place, int j) {
+        constexpr int R = decltype(place)::value;
+        constexpr int kK = ((R + 1) & 3) * 16384, kV = R * 16384, kN = ((R + 2) & 3) * 16384;
+        bf16x8_t vf[16];
+        uint32_t pw[16];  // packed weights, two per word
+        float y[33], x[34];
+        f32x4_t rs = {0.0f, 0.0f, 0.0f, 0.0f};
+        auto stage = [&](int e) {  // e = 0 .. 34
+            if (e >= 6 && (e & 3) == 2) rs = add_weights(pw[(e - 6) >> 1], pw[((e - 6) >> 1) + 1], rs);
+            if (e >= 3 && (e & 1) && e < 34) {
+                const f32x2_t pr = {x[e - 3], x[e - 2]};
+                pw[(e - 3) >> 1] = __builtin_bit_cast(uint32_t, __builtin_convertvector(pr, bf16x2_t));
             }
+            if (e >= 1 && e <= 32) x[e - 1] = __builtin_amdgcn_exp2f(y[e - 1]);
+            if (e < 32) y[e] = __builtin_fmaf(sc[e >> 4][e & 15], sl2, m_neg);
+        };
+        auto pf = [&](int s4) {
+            const u32x4_t v = {pw[4 * s4], pw[4 * s4 + 1], pw[4 * s4 + 2], pw[4 * s4 + 3]};
+            return __builtin_bit_cast(bf16x8_t, v);
+        };
+        const f32x16_t zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+        constexpr int kEarly = 6;  // groups with two stages
+        int e = 0;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            if (i + kAhead < 16) kf[i + kAhead] = k_frag(kK, i + kAhead);
+            if (i >= 16 - kVAhead) vf[i - 16 + kVAhead] = v_frag(kV, i - 16 + kVAhead);
+            sn[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[i], qf[i >> 1], i < 2 ? zero : sn[i & 1], 0, 0, 0);
+            stage(e++);
+            if (i < kEarly) stage(e++);
+            asm volatile("" : "+v"(sn[i & 1]), "+v"(y[e - 1]), "+v"(x[e - 2]), "+v"(rs), "+v"(sc[e >> 4]) : : "memory");
+            __builtin_amdgcn_sched_barrier(0);
         }
+        mid_slot();
+        const Blk nb = next_blk(j + 5);
+        float mx = -__builtin_inff();
+        bool up = false;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            if (i + kVAhead < 16) vf[i + kVAhead] = v_frag(kV, i + kVAhead);
+            if (i >= 16 - kAhead) kf[i - 16 + kAhead] = k_frag(kN, i - 16 + kAhead);
+            oacc[i & 3] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[i], pf(i >> 2), oacc[i & 3], 0, 0, 0);
+            if (e < 35) {
+                stage(e++);
+                if (e < 33) asm volatile("" : "+v"(y[e - 1]) : : "memory");
+                if (e < 34) asm volatile("" : "+v"(x[e - 2]) : : "memory");
+                asm volatile("" : "+v"(rs), "+v"(sc[1]) : : "memory");
+            }
+            if (i >= 4 && i < 12) {  // the row max of the next block's 32 scores
+                const int u = i - 4;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) mx = fmaxf(mx, sn[u >> 2][4 * (u & 3) + q]);
+            }
+            if (i == 12) mx = xor32_max(mx) * sl2;
+            if (i == 13) up = __ballot(mx > m_run + kRescale) != 0;
+            if (i == 14) l_run += rs[0];  // this lane's half of the row; combined across lanes n, n+32 at the end
+            asm volatile("" : "+v"(oacc[i & 3]), "+v"(mx), "+v"(l_run) : : "memory");
+            if (i == 1) issue_v(j + 3, 0, vq0);
+            if (i == 4) issue_v(j + 3, 1, vq0);
+            if (i == 7) issue_k(j + 5, 0, nb);
+            if (i == 10) issue_k(j + 5, 1, nb);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        vq0 = vq1;
+        vq1 = nb;
+        if (up) rise(mx);
     };
 
-    // ---- KV loop: four LDS stages, DMA three blocks ahead ----
-    const int nblk = e1 - e0;
-    for (int i = 0; i < 3; ++i)
-        if (i < nblk) issue_block(e0 + i, i);
-    // block 0 must have landed (4 loads per block and wave)
-    if (nblk > 2) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-    else if (nblk > 1) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-    else wait_dma();
-    __syncthreads();
-    auto step = [&](int idx, bool masked) {
-        if (idx + 3 < nblk) issue_block(e0 + idx + 3, (idx + 3) % kStages);
-        process(block_id(e0 + idx), smem + (idx % kStages) * kStageBytes, masked);
-        // block idx+1 must have landed; later blocks may stay in flight
-        if (idx + 3 < nblk) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-        else if (idx + 2 < nblk) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-        else wait_dma();
+    const int n_un = e_mask - e0;  // blocks before the first masked one
+    if (nblk > 0) {
+        next = load_blks(0);
+        const Blk b0 = next_blk(0), b1 = next_blk(1);
+        vq0 = next_blk(2);
+        vq1 = next_blk(3);
+        for (int half = 0; half < 2; ++half) issue_k(0, half, b0);
+        for (int half = 0; half < 2; ++half) issue_k(1, half, b1);
+        for (int half = 0; half < 2; ++half) issue_v(0, half, b0);
+        for (int half = 0; half < 2; ++half) issue_k(2, half, vq0);
+        for (int half = 0; half < 2; ++half) issue_v(1, half, b1);
+        for (int half = 0; half < 2; ++half) issue_k(3, half, vq1);
+        asm volatile("s_waitcnt vmcnt(10)" ::: "memory");
         __syncthreads();
-    };
-    int idx = 0;
-    for (; idx < e_mask - e0; ++idx) step(idx, false);
-    for (; idx < nblk; ++idx) step(idx, true);
+        scores(0);
+        if (n_un == 0) mask(block_id(e0));
+        block_max();
+        mid_slot();
+        issue_slot(-1);
+        int j = 0;
+        f32x16_t sn[2];
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) kf[i] = k_frag(16384, i);
+        // four slots a round: the ring places are constants and the scores change places
+        // without copies
+        for (; j + 4 < n_un; j += 4) {
+            fused(sc, sn, IntC<0>{}, j);
+            fused(sn, sc, IntC<1>{}, j + 1);
+            fused(sc, sn, IntC<2>{}, j + 2);
+            fused(sn, sc, IntC<3>{}, j + 3);
+        }
+        if (j + 2 < n_un) {
+            fused(sc, sn, IntC<0>{}, j);
+            fused(sn, sc, IntC<1>{}, j + 1);
+            j += 2;
+        }
+        for (; j < nblk; ++j) {  // the next block is masked, or there is none
+            finish((j & 3) * 16384);
+            if (j + 1 < nblk) {
+                scores(((j + 1) & 3) * 16384);
+                if (j + 1 >= n_un) mask(block_id(e0 + j + 1));
+                block_max();
+                mid_slot();
+                issue_slot(j);
+            }
+        }
+        wait_dma();  // no load may write LDS after the workgroup has ended
+    }
 
     // ---- epilogue ----
     // lanes n and n + 32 hold different keys of the same row: their partial sums combine
@@ -1108,19 +1273,22 @@ hipError_t launch_attn(const AttnArgs& a, hipStream_t stream) {
     p.ws_unsplit = plan.max > 1 && plan.may_unsplit && a.table
                        ? reinterpret_cast<int32_t*>(p.ws_lse + (int64_t)plan.max * rows_all)
                        : nullptr;
+    bool row_res;
     {
         int max_tokens = 0;
         for (int b = 0; b < a.s.B; ++b) max_tokens = max(max_tokens, p.qpos0[b] + a.s.Lq);
         const int64_t stok = max(a.k.stok, a.v.stok);
-        p.row_res = a.k.page_table == nullptr && a.v.page_table == nullptr && a.k.sblk == 64 * a.k.stok &&
+        row_res = a.k.page_table == nullptr && a.v.page_table == nullptr && a.k.sblk == 64 * a.k.stok &&
                     a.v.sblk == 64 * a.v.stok && (int64_t)max_tokens * stok * 2 + 64 * stok * 2 < (int64_t{1} << 31);
     }
+    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(p.per_xcd * 8), dim3(kNW * 64), 0, stream, p); };
+    static_assert(kNW == kDecWaves, "one workgroup size for the attention kernels");
     if (a.table)
-        hipLaunchKernelGGL((attn_fwd_kernel<kNW, true>), dim3(p.per_xcd * 8), dim3(kNW * 64), 0, stream, p);
+        row_res ? launch(attn_fwd_kernel<kNW, true, true>) : launch(attn_fwd_kernel<kNW, true, false>);
     else if (attn_uses_decode_kernel(a.s, true))
-        hipLaunchKernelGGL(attn_decode_kernel, dim3(p.per_xcd * 8), dim3(kDecWaves * 64), 0, stream, p);
+        launch(attn_decode_kernel);
     else
-        hipLaunchKernelGGL((attn_fwd_kernel<kNW, false>), dim3(p.per_xcd * 8), dim3(kNW * 64), 0, stream, p);
+        row_res ? launch(attn_fwd_kernel<kNW, false, true>) : launch(attn_fwd_kernel<kNW, false, false>);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || plan.max <= 1) return e;
     const int64_t blocks = (rows_all + 7) / 8;
