@@ -72,6 +72,7 @@ struct AttnParams {
     SeqAddr out;
     float* lse;
     int ntiles;       // packed-row tiles per KV row
+    int sp0;          // splits of the first request (of every one in kPlaceRows and kPlaceSplits)
     int rows_total;   // Lq * G
     int total_items;  // B*Hkv*ntiles*splits
     int per_xcd;      // ceil(total_items / 8)
@@ -85,12 +86,81 @@ struct AttnParams {
     int32_t nkb[CA_MAX_BATCH];       // valid logical blocks of each request
     int32_t sp[CA_MAX_BATCH];        // splits of each request's block lists
     int32_t ioff[CA_MAX_BATCH + 1];  // first work item of each request (linear placement)
-    int use_rows;                    // units placed per XCD (xoff / xrow / xlo / xcnt)
-    int32_t xoff[9];
-    uint16_t xrow[kPlanRows];
-    uint8_t xlo[kPlanRows];
-    uint8_t xcnt[kPlanRows];
+    int placement;                   // kPlace*: where a workgroup finds its unit
+    int units;                       // kPlaceSplits: units in all
+    int32_t xoff[9];                 // kPlaceTable
+    uint32_t unit[kPlanRows];
 };
+
+// The work item of a workgroup: KV row, request, split of the row's list (of p.sp[b]) and, for
+// kernels with row tiles, the tile.
+struct Item {
+    int row, b, split, tile;
+};
+// Workgroup L runs on XCD L % 8 and is that XCD's (L / 8)-th; false when the XCD has no such
+// item.  Equal requests need no table (kPlaceRows, kPlaceSplits: arithmetic); a ragged launch's
+// units are read 64 at a time, one per lane, and found by a prefix sum over their items, so the
+// search costs one read's latency and not one per unit.
+__device__ __forceinline__ bool find_item(const AttnParams& p, int ntiles, Item* it) {
+    const int x = blockIdx.x & 7;
+    int k = blockIdx.x >> 3;
+    const int Hkv = p.s.Hkv;
+    int lo = 0, cnt;
+    if (p.placement == kPlaceRows) {
+        cnt = p.sp0;
+        const int u = k / (ntiles * cnt);
+        it->row = x + 8 * u;
+        if (it->row >= p.s.B * Hkv) return false;
+        k -= u * ntiles * cnt;
+    } else if (p.placement == kPlaceSplits) {
+        cnt = 1;
+        const int u = x + 8 * (k / ntiles);
+        if (u >= p.units) return false;
+        it->row = u / p.sp0;
+        lo = u - it->row * p.sp0;
+        k %= ntiles;
+    } else if (p.placement == kPlaceTable) {
+        const int lane = threadIdx.x & 63;
+        const int end = p.xoff[x + 1];
+        int base = p.xoff[x];
+        uint32_t word = 0;
+        for (;; base += 64) {
+            if (base >= end) return false;
+            const uint32_t w = base + lane < end ? p.unit[base + lane] : 0u;
+            int sum = ntiles * static_cast<int>(w >> 24);  // inclusive prefix of the units' items
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const int y = __shfl_up(sum, o, 64);
+                if (lane >= o) sum += y;
+            }
+            const int total = __builtin_amdgcn_readlane(sum, 63);
+            if (k < total) {
+                const int u = __popcll(__ballot(sum <= k));
+                word = __builtin_amdgcn_readlane(w, u);
+                if (u > 0) k -= __builtin_amdgcn_readlane(sum, u - 1);
+                break;
+            }
+            k -= total;
+        }
+        it->row = word & 0xffffu;
+        lo = (word >> 16) & 0xffu;
+        cnt = word >> 24;
+    } else {
+        const int W = x * p.per_xcd + k;
+        if (W >= p.total_items) return false;
+        int b = 0;
+        while (b + 1 < p.s.B && p.ioff[b + 1] <= W) ++b;
+        cnt = p.sp[b];
+        const int local = W - p.ioff[b];
+        const int u = local / (ntiles * cnt);
+        it->row = b * Hkv + u;
+        k = local - u * ntiles * cnt;
+    }
+    it->b = it->row / Hkv;
+    it->tile = k / cnt;
+    it->split = lo + k - it->tile * cnt;
+    return true;
+}
 
 __device__ __forceinline__ int swap23(int m) {
     return (m & ~12) | ((m & 4) << 1) | ((m & 8) >> 1);
@@ -191,58 +261,33 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
     }
 
     // workgroup -> (XCD x, k-th work item of x) -> (KV row, row tile, split)
-    const int L = blockIdx.x;
-    const int x = L & 7;
-    int k = L >> 3;
     const Shape& s = p.s;
-    int row, b, split, tile;
-    if (p.use_rows && kTab && unsplit) {
+    Item it;
+    if (kTab && unsplit) {
         // an unsplit launch takes the XCD's items split-major (its units are whole rows with
         // one split count): the items of split 0 of every unit first, so the working items are
         // dispatched first and the idle ones after them (interleaved, the idle items held the
-        // working ones back: 510 vs 290 us on config 4); a split launch keeps the unit-major
-        // order below, which runs a long row's items before a short row's
+        // working ones back: 510 vs 290 us on a four-request ragged batch); a split launch
+        // keeps the unit-major order, which runs a long row's items before a short row's
+        const int x = blockIdx.x & 7;
+        const int k = blockIdx.x >> 3;
         const int i0 = p.xoff[x];
         const int per = (p.xoff[x + 1] - i0) * p.ntiles;  // items of one split on this XCD
-        if (per == 0) return;
-        const int sidx = k / per;
-        const int kk = k - sidx * per;
-        const int i = i0 + kk / p.ntiles;
-        if (sidx >= p.xcnt[i]) return;
-        row = p.xrow[i];
-        b = row / s.Hkv;
-        split = p.xlo[i] + sidx;
-        tile = kk - (kk / p.ntiles) * p.ntiles;
-    } else if (p.use_rows) {
-        int i = p.xoff[x];
-        const int iend = p.xoff[x + 1];
-        for (; i < iend; ++i) {
-            const int items = p.ntiles * p.xcnt[i];
-            if (k < items) break;
-            k -= items;
-        }
-        if (i >= iend) return;
-        row = p.xrow[i];
-        b = row / s.Hkv;
-        split = p.xlo[i] + k % p.xcnt[i];
-        tile = k / p.xcnt[i];
-    } else {
-        const int W = x * p.per_xcd + k;
-        if (W >= p.total_items) return;
-        b = 0;
-        while (b + 1 < s.B && p.ioff[b + 1] <= W) ++b;
-        const int per_row = p.ntiles * p.sp[b];
-        row = b * s.Hkv + (W - p.ioff[b]) / per_row;
-        const int local = (W - p.ioff[b]) % per_row;
-        split = local % p.sp[b];
-        tile = local / p.sp[b];
+        if (k >= per) return;  // the unsplit row's items are those of split 0
+        const int i = k / p.ntiles;
+        it.row = p.unit[i0 + i] & 0xffffu;
+        it.b = it.row / s.Hkv;
+        it.split = 0;
+        it.tile = k - i * p.ntiles;
+    } else if (!find_item(p, p.ntiles, &it)) {
+        return;
     }
+    const int row = __builtin_amdgcn_readfirstlane(it.row);
+    const int b = __builtin_amdgcn_readfirstlane(it.b);
+    const int split = __builtin_amdgcn_readfirstlane(it.split);
+    const int tile = __builtin_amdgcn_readfirstlane(it.tile);
     const int hk = row - b * s.Hkv;
-    int nsplit = p.sp[b];
-    if (unsplit) {
-        if (split != 0) return;
-        nsplit = 1;
-    }
+    const int nsplit = unsplit ? 1 : p.sp[b];
     const int G = s.G;
     const int qpos0 = p.qpos0[b];  // query row t sits at absolute position qpos0 + t
     const int nkb = p.nkb[b];      // valid logical block ids are [0, nkb)
@@ -256,27 +301,13 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
     const int32_t* tab = kTab ? p.table + (int64_t)row * p.table_stride : nullptr;
     auto block_id = [&](int e) { return kTab ? min(max(sload(tab + e), 0), nkb - 1) : e; };
     const int lim = (qpos0 + t_last) >> 6;  // last block the tile can see
-    int n_vis;
-    if (kTab) {
-        n_vis = min(max(sload(p.counts + row), 0), s.cap);
-        while (n_vis > 0 && sload(tab + n_vis - 1) > lim) --n_vis;
-    } else {
-        n_vis = min(nkb, lim + 1);
-    }
-    const int chunk = (n_vis + nsplit - 1) / nsplit;
-    const int e0 = min(n_vis, split * chunk);
-    const int e1 = min(n_vis, e0 + chunk);
-    // entries at or after e_mask contain keys beyond the tile's first query position
-    int e_mask = e1;
-    while (e_mask > e0 && block_id(e_mask - 1) * 64 + 63 > qpos0 + t_first) --e_mask;
-
     const int tid = threadIdx.x;
     const int w = tid >> 6;
     const int l = tid & 63;
     const int h = l >> 5;
     const int n = l & 31;
 
-    // ---- Q fragments (B operand of S^T = K Q^T) ----
+    // ---- Q fragments (B operand of S^T = K Q^T); the loads are in flight while the lists are read ----
     const int qrow = r0 + 32 * w + n;
     const bool qvalid = qrow < rows_total;
     const int qt = qvalid ? qrow / G : 0;
@@ -294,6 +325,43 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
             }
         }
     }
+    // (and so is a read of the list's first lines and page, which the ids below need)
+    const int warm = kTab && l < s.cap ? tab[l] : 0;
+    CA_PIN();
+    // n_vis: entries up to the last one the tile can see; n_whole: entries whose blocks hold no key
+    // beyond the tile's first query position (blocks [0, whole)).  The lists ascend and end in
+    // the chunk's own blocks, so both usually lie in the last 64 entries: one read, a lane each.
+    const int whole = (qpos0 + t_first + 1) >> 6;
+    int n_vis, n_whole;
+    if (kTab) {
+        int end = min(max(sload(p.counts + row), 0), s.cap);
+        n_vis = -1;
+        for (;; end -= 64) {
+            const int e = end - 1 - l;
+            const int id = e >= 0 ? tab[e] : -1;
+            if (n_vis < 0) {
+                const uint64_t seen = __ballot(id <= lim);
+                if (seen == 0) continue;
+                n_vis = max(0, end - (__ffsll(static_cast<unsigned long long>(seen)) - 1));
+            }
+            const uint64_t low = __ballot(min(id, nkb - 1) < whole);
+            if (low) {
+                n_whole = max(0, end - (__ffsll(static_cast<unsigned long long>(low)) - 1));
+                break;
+            }
+        }
+    } else {
+        n_vis = min(nkb, lim + 1);
+        n_whole = whole;
+    }
+    const int chunk = (n_vis + nsplit - 1) / nsplit;
+    const int e0 = min(n_vis, split * chunk);
+    const int e1 = min(n_vis, e0 + chunk);
+    // entries at or after e_mask contain keys beyond the tile's first query position
+    const int e_mask = min(max(n_whole, e0), e1);
+    const int nblk = e1 - e0;
+    asm volatile("" : : "v"(warm));
+
     const int qtok = qvalid ? qt : 0x3fffffff;
 
     f32x16_t oacc[4];
@@ -380,6 +448,8 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
         }
         return b;
     };
+
+    if (nblk > 0) next = load_blks(0);
 
     const float sl2 = p.scale_log2;
 
@@ -497,7 +567,6 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
     // block j + 5 after it, into the places of those two in rings of four blocks, and the
     // loads stay in flight for two (V) and three (K) slots.  Every slot issues its four loads
     // (blocks past the list's end load nothing), so the counts of the waits are constants.
-    const int nblk = e1 - e0;
     Blk vq0, vq1;  // the two entries whose K is issued and V is not
     auto issue_k = [&](int i, int half, const Blk& b) {
         load_half(kbase_row, k_rsrc, p.k.sblk, kstok_b, k_goff, b.id, b.kp, half, lds0 + (i & 3) * 16384);
@@ -598,7 +667,6 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
 
     const int n_un = e_mask - e0;  // blocks before the first masked one
     if (nblk > 0) {
-        next = load_blks(0);
         const Blk b0 = next_blk(0), b1 = next_blk(1);
         vq0 = next_blk(2);
         vq1 = next_blk(3);
@@ -781,32 +849,12 @@ constexpr int kDecOStride = 132;  // floats per row of a wave's partial O in LDS
 __global__ __launch_bounds__(kDecWaves * 64) void attn_decode_kernel(AttnParams p) {
     __shared__ __attribute__((aligned(16))) uint8_t smem[kDecWaves * kDecVBytes];
 
-    const int L = blockIdx.x;
-    const int x = L & 7;
-    int k = L >> 3;
     const Shape& s = p.s;
-    int row, b, split;
-    if (p.use_rows) {
-        int i = p.xoff[x];
-        const int iend = p.xoff[x + 1];
-        for (; i < iend; ++i) {
-            const int items = p.xcnt[i];
-            if (k < items) break;
-            k -= items;
-        }
-        if (i >= iend) return;
-        row = p.xrow[i];
-        b = row / s.Hkv;
-        split = p.xlo[i] + k;
-    } else {
-        const int W = x * p.per_xcd + k;
-        if (W >= p.total_items) return;
-        b = 0;
-        while (b + 1 < s.B && p.ioff[b + 1] <= W) ++b;
-        const int per_row = p.sp[b];
-        row = b * s.Hkv + (W - p.ioff[b]) / per_row;
-        split = (W - p.ioff[b]) % per_row;
-    }
+    Item it;
+    if (!find_item(p, 1, &it)) return;
+    const int row = __builtin_amdgcn_readfirstlane(it.row);
+    const int b = __builtin_amdgcn_readfirstlane(it.b);
+    const int split = __builtin_amdgcn_readfirstlane(it.split);
     const int hk = row - b * s.Hkv;
     const int nsplit = p.sp[b];
     const int G = s.G;
@@ -1115,11 +1163,11 @@ void attn_plan(const Shape& s, const int32_t* nkb, int forced, bool dense, Split
         plan->off[b + 1] = plan->off[b] + s.Hkv * ntiles * sb;
     }
     const int rows = s.B * s.Hkv;
-    plan->use_rows = rows <= kPlanRows;
-    if (!plan->use_rows) {
-        plan->per_xcd = (plan->off[s.B] + 7) / 8;
-        return;
-    }
+    plan->sp0 = plan->s[0];
+    plan->placement = kPlaceLinear;
+    plan->units = 0;
+    plan->per_xcd = (plan->off[s.B] + 7) / 8;
+    if (rows > kPlanRows) return;
     // Placement units on the 8 XCDs.  A unit is a KV row and a range of its splits; the row
     // tiles of a unit stream the same blocks, so they share the XCD's L2, and different
     // split ranges of a row are disjoint parts of its block list (placing them apart
@@ -1136,6 +1184,14 @@ void attn_plan(const Shape& s, const int32_t* nkb, int forced, bool dense, Split
     for (int r = 0; r < rows; ++r) nunits += plan->s[r / s.Hkv];
     // (a launch that may run unsplit keeps whole rows: each XCD's tiles then fit one round)
     const bool split_units = (rows % 8 != 0 || !same_len) && nunits <= kPlanRows && !plan->may_unsplit;
+    // requests of one length: unit u on XCD u % 8 in both cases, by arithmetic in the kernel
+    if (same_len && (rows % 8 == 0 || split_units)) {
+        plan->placement = split_units ? kPlaceSplits : kPlaceRows;
+        plan->units = split_units ? nunits : rows;
+        plan->per_xcd = (plan->units + 7) / 8 * ntiles * (split_units ? 1 : plan->sp0);
+        return;
+    }
+    plan->placement = kPlaceTable;
     int unit_row[kPlanRows], unit_lo[kPlanRows], unit_cnt[kPlanRows];
     double unit_work[kPlanRows];  // blocks x row tiles the unit's items stream
     int units = 0;
@@ -1198,9 +1254,7 @@ void attn_plan(const Shape& s, const int32_t* nkb, int forced, bool dense, Split
     for (int x = 0; x < 8; ++x) {
         for (int i = 0; i < nunit[x]; ++i) {
             const int u = lists[x][i];
-            plan->xrow[plan->xoff[x] + i] = static_cast<uint16_t>(unit_row[u]);
-            plan->xlo[plan->xoff[x] + i] = static_cast<uint8_t>(unit_lo[u]);
-            plan->xcnt[plan->xoff[x] + i] = static_cast<uint8_t>(unit_cnt[u]);
+            plan->unit[plan->xoff[x] + i] = static_cast<uint32_t>(unit_row[u] | unit_lo[u] << 16 | unit_cnt[u] << 24);
         }
         plan->xoff[x + 1] = plan->xoff[x] + nunit[x];
         plan->per_xcd = max(plan->per_xcd, items[x]);
@@ -1259,13 +1313,12 @@ hipError_t launch_attn(const AttnArgs& a, hipStream_t stream) {
     for (int b = 0; b <= CA_MAX_BATCH; ++b) p.ioff[b] = b <= a.s.B ? plan.off[b] : plan.off[a.s.B];
     p.total_items = plan.off[a.s.B];
     p.per_xcd = plan.per_xcd;
-    p.use_rows = plan.use_rows;
-    for (int x = 0; x < 9; ++x) p.xoff[x] = plan.use_rows ? plan.xoff[x] : 0;
-    for (int i = 0; i < kPlanRows; ++i) {
-        const bool used = plan.use_rows && i < plan.xoff[8];
-        p.xrow[i] = used ? plan.xrow[i] : 0;
-        p.xlo[i] = used ? plan.xlo[i] : 0;
-        p.xcnt[i] = used ? plan.xcnt[i] : 1;
+    p.placement = plan.placement;
+    p.sp0 = plan.sp0;
+    p.units = plan.units;
+    if (plan.placement == kPlaceTable) {  // the kernels read the table in this case only
+        for (int x = 0; x < 9; ++x) p.xoff[x] = plan.xoff[x];
+        for (int i = 0; i < plan.xoff[8]; ++i) p.unit[i] = plan.unit[i];
     }
     const int64_t rows_all = (int64_t)a.s.B * a.s.Hkv * p.rows_total;
     p.ws_o = plan.max > 1 ? static_cast<float*>(a.workspace) : nullptr;

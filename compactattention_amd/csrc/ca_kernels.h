@@ -103,25 +103,27 @@ constexpr int kMaxPrefillSplits = 16;
 constexpr int kMaxDecodeSplits = 64;
 
 // Split-KV plan.  Request b's block lists are cut into s[b] pieces (max = the largest,
-// which sizes the workspace).  Work placement: with at most kPlanRows KV rows, whole rows
-// go to XCDs (longest first, each to the least-loaded XCD), so a row's items share one L2
-// and the XCDs carry equal work: entries xoff[x] .. xoff[x+1] list XCD x's units in order,
-// each a row (xrow) and a range of its splits (xlo, xcnt).  When the rows do not divide
-// evenly over the XCDs, each split of a row is a unit of its own, so the XCDs' loads even
-// out; its items stream a disjoint part of the row's block list.
-// Otherwise items are numbered request by request (off[b]) and dealt to XCDs in
-// contiguous ranges.
+// which sizes the workspace).  Work placement (placement):
+//  - kPlaceRows: requests of one length whose rows divide over the 8 XCDs: KV row r on XCD r % 8,
+//    so a row's items share one L2 and the XCDs carry equal work;
+//  - kPlaceSplits: requests of one length otherwise: split u % sp0 of row u / sp0 on XCD u % 8
+//    (a row's splits stream disjoint parts of its block list);
+//  - kPlaceTable: ragged launches: entries xoff[x] .. xoff[x+1] list XCD x's units in order, each
+//    a row and a range of its splits (unit: row | first split << 16 | splits << 24);
+//  - kPlaceLinear: more than kPlanRows KV rows: items numbered request by request (off[b]) and
+//    dealt to XCDs in contiguous ranges.
 constexpr int kPlanRows = 512;
+enum { kPlaceLinear = 0, kPlaceRows = 1, kPlaceSplits = 2, kPlaceTable = 3 };
 struct SplitPlan {
     int32_t s[CA_MAX_BATCH];
     int32_t off[CA_MAX_BATCH + 1];
     int max;
-    int use_rows;
+    int placement;
+    int sp0;          // splits of the first request
+    int units;        // kPlaceRows, kPlaceSplits
     int per_xcd;      // work items per XCD (grid = 8 * per_xcd)
     int may_unsplit;  // the kernel drops the splits when the rows' selected counts are even
-    uint16_t xrow[kPlanRows];  // placement units: a row and a range of its splits
-    uint8_t xlo[kPlanRows];    // first split of the unit
-    uint8_t xcnt[kPlanRows];   // splits in the unit
+    uint32_t unit[kPlanRows];
     int32_t xoff[9];
 };
 
