@@ -17,6 +17,8 @@
 // Every reduction that feeds a selection decision runs in a fixed order (see ca_common.h),
 // so the scores and tables equal a sequential CPU evaluation bit for bit.
 
+#include <type_traits>
+
 #include "ca_common.h"
 #include "ca_kernels.h"
 
@@ -261,30 +263,32 @@ __global__ __launch_bounds__(256) void chunk_summaries_kernel(Shape s, SeqAddr k
 // ---------------------------------------------------------------------------------------
 // Block logits: logits[(b*Hq + h)*Qb + qb][kb] = dot(qhat[b,h,qb], khat[b, h/G, kb]) * scale
 // for the causal kb <= P + qb.  The G*Qb query vectors of a KV group are contiguous in
-// qhat, so a workgroup takes a 64 (query vectors) x KT (key blocks) tile of one group;
-// each thread owns a 4 x KT/16 register tile and every dot product is one sequential fma
-// chain over d = 0..127.
+// qhat, so a workgroup takes a tile of 16 NQ query vectors x 64 key blocks of one group.
+//
+// Every dot product is one sequential fma chain over d = 0..127, on the matrix cores: the fp32
+// MFMAs with one product per element and instruction round like fma (bit for bit, subnormals,
+// infinities and NaN included), so the order of a chain is the order of the instructions.  The
+// 4x4x1 form (16 blocks) runs 54 products a cycle and SIMD where four chains alternate, the
+// 16x16x1 one 32 and fmas 16; a step of a wave's 32 x 32 logits reads four floats a lane from
+// LDS.  Few query vectors take a wave of 16 x 64.
+// Bound by latency (launch, loads, 512 MFMAs a wave): kernel times against 4 x 2 register tiles of
+// fmas, 64 vectors x 2064 keys x 8 groups 11.7 -> 11.5 us, 56 x 2056 x 16 ragged 12.0 -> 11.0,
+// 32 x 1032 x 8 8.5 -> 6.9, 16 x 128 x 8 6.4 -> 6.2.
 constexpr int kPadRow = kD + 4;  // LDS row pitch (floats) for summary tiles
-constexpr int kLogitsGridSlots = 512;  // block-logits workgroups resident at once (2 per CU)
+constexpr int kLogitsKeys = 64;  // key blocks per workgroup
 
-// One workgroup computes a 64-row x KT-key tile of logits (KT = 32: twice the workgroups of
-// 64-key tiles, so the last round of the grid carries half as much work per CU).  The first
-// `extra` tiles of a row hold one key more (tile x starts at KT x + min(x, extra)): a row
-// whose keys need just over a multiple of two workgroups per CU stays in one round of the
-// grid instead of spilling a few tiles into a second (config 2: 2064 keys per row as 64
-// tiles, 16 of them of 33 keys).  Wave 0 computes the extra key's 64 logits, one fma chain
-// per row in the same order.
-template <int KT>
-__global__ __launch_bounds__(256) void block_logits_kernel(Shape s, const float* qhat, const float* khat,
-                                                           float scale, PastBlocks pb, float* logits, int extra) {
-    static_assert(KT == 32 || KT == 64, "16 key groups of KT/16 keys");
-    constexpr int KJ = KT / 16;  // keys per thread
-    __shared__ __attribute__((aligned(16))) float qt[64 * kPadRow];
-    __shared__ __attribute__((aligned(16))) float kt[(KT + 1) * kPadRow];
-    const int kb0 = blockIdx.x * KT + min((int)blockIdx.x, extra);
-    const bool has_extra = (int)blockIdx.x < extra;
+typedef float f32x4_v __attribute__((ext_vector_type(4)));
+
+template <int NQ>
+__global__ __launch_bounds__(64 * NQ) void block_logits_kernel(Shape s, const float* qhat, const float* khat,
+                                                               float scale, PastBlocks pb, float* logits) {
+    static_assert(NQ == 1 || NQ == 2 || NQ == 4, "one, two or four waves");
+    constexpr int QR = 16 * NQ;  // query vectors of the workgroup
+    __shared__ __attribute__((aligned(16))) float qt[QR * kPadRow];
+    __shared__ __attribute__((aligned(16))) float kt[kLogitsKeys * kPadRow];
+    const int kb0 = blockIdx.x * kLogitsKeys;
     const int row = blockIdx.y;
-    const int m0 = blockIdx.z * 64;
+    const int m0 = blockIdx.z * QR;
     const int b = row / s.Hkv;
     const int hk = row - b * s.Hkv;
     const int P = pb.p[b];
@@ -294,99 +298,82 @@ __global__ __launch_bounds__(256) void block_logits_kernel(Shape s, const float*
     const int t = threadIdx.x;
     const float* qbase = qhat + ((int64_t)(b * s.Hq + hk * s.G) * s.Qb + m0) * kD;
     const float* kbase = khat + ((int64_t)row * s.cap + kb0) * kD;
-    const int mrows = min(64, M - m0);
-    const int krows = min(KT + (has_extra ? 1 : 0), nkb - kb0);
+    const int mrows = min(QR, M - m0);
+    const int krows = min(kLogitsKeys, nkb - kb0);
     {
-        // all loads of a thread in flight before the LDS stores
-        constexpr int kQIters = 64 * (kD / 4) / 256;
-        constexpr int kKIters = KT * (kD / 4) / 256;
-        float4 qv[kQIters], kv[kKIters];
         // unconditional loads (rows past the tile's last valid row re-read that row; their
-        // logits are computed and never stored), so all of them are in flight at once
+        // logits are computed and never stored), all in flight before the LDS stores
+        constexpr int kThreads = 64 * NQ;
+        constexpr int kQIters = QR * (kD / 4) / kThreads;
+        constexpr int kKIters = kLogitsKeys * (kD / 4) / kThreads;
+        float4 qv[kQIters], kv[kKIters];
 #pragma unroll
         for (int i = 0; i < kQIters; ++i) {
-            const int f = t + 256 * i;
-            const int r = f >> 5, c4 = f & 31;
-            qv[i] = *reinterpret_cast<const float4*>(qbase + (int64_t)min(r, mrows - 1) * kD + c4 * 4);
+            const int f = t + kThreads * i;
+            qv[i] = *reinterpret_cast<const float4*>(qbase + (int64_t)min(f >> 5, mrows - 1) * kD + (f & 31) * 4);
         }
 #pragma unroll
         for (int i = 0; i < kKIters; ++i) {
-            const int f = t + 256 * i;
-            const int r = f >> 5, c4 = f & 31;
-            kv[i] = *reinterpret_cast<const float4*>(kbase + (int64_t)min(r, krows - 1) * kD + c4 * 4);
+            const int f = t + kThreads * i;
+            kv[i] = *reinterpret_cast<const float4*>(kbase + (int64_t)min(f >> 5, krows - 1) * kD + (f & 31) * 4);
         }
 #pragma unroll
         for (int i = 0; i < kQIters; ++i) {
-            const int f = t + 256 * i;
-            const int r = f >> 5, c4 = f & 31;
-            *reinterpret_cast<float4*>(qt + r * kPadRow + c4 * 4) = qv[i];
+            const int f = t + kThreads * i;
+            *reinterpret_cast<float4*>(qt + (f >> 5) * kPadRow + (f & 31) * 4) = qv[i];
         }
 #pragma unroll
         for (int i = 0; i < kKIters; ++i) {
-            const int f = t + 256 * i;
-            const int r = f >> 5, c4 = f & 31;
-            *reinterpret_cast<float4*>(kt + r * kPadRow + c4 * 4) = kv[i];
+            const int f = t + kThreads * i;
+            *reinterpret_cast<float4*>(kt + (f >> 5) * kPadRow + (f & 31) * 4) = kv[i];
         }
-        if (has_extra && t < 32)  // key KT of the tile (re-read of the last valid row past nkb)
-            *reinterpret_cast<float4*>(kt + KT * kPadRow + t * 4) =
-                *reinterpret_cast<const float4*>(kbase + (int64_t)min(KT, krows - 1) * kD + t * 4);
     }
     __syncthreads();
+    // The wave's 16 CQ query vectors x 16 CK keys: MFMA (cq, ck) holds 16 x 16 of them as 4 x 4
+    // blocks of 4 x 4, block b = lane / 4 at query rows 4 (b % 4), keys 4 (b / 4).
+    constexpr int CQ = NQ == 1 ? 1 : 2, CK = 4 / CQ;
     const int lane = t & 63;
-    const int tm = lane & 15;              // query rows tm + 16 i
-    const int tn = (t >> 6) * 4 + (lane >> 4);  // key rows KJ tn + j
-    float acc[4][KJ];
+    const int w = t >> 6;
+    const int wq = NQ == 4 ? 32 * (w >> 1) : 0;
+    const int wk = NQ == 1 ? 0 : 32 * (w & 1);
+    const int bq = 4 * ((lane >> 2) & 3), bk = 4 * (lane >> 4), n = lane & 3;
+    const float* qa = qt + (wq + bq + n) * kPadRow;
+    const float* ka = kt + (wk + bk + n) * kPadRow;
+    f32x4_v acc[CQ][CK];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < CQ; ++i)
 #pragma unroll
-        for (int j = 0; j < KJ; ++j) acc[i][j] = 0.0f;
+        for (int j = 0; j < CK; ++j) acc[i][j] = f32x4_v{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 8
     for (int d = 0; d < kD; d += 4) {
-        float4 a[4], c[KJ];
+        f32x4_v a[CQ], c[CK];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) a[i] = *reinterpret_cast<const float4*>(qt + (tm + 16 * i) * kPadRow + d);
+        for (int i = 0; i < CQ; ++i) a[i] = *reinterpret_cast<const f32x4_v*>(qa + 16 * i * kPadRow + d);
 #pragma unroll
-        for (int j = 0; j < KJ; ++j) c[j] = *reinterpret_cast<const float4*>(kt + (KJ * tn + j) * kPadRow + d);
+        for (int j = 0; j < CK; ++j) c[j] = *reinterpret_cast<const f32x4_v*>(ka + 16 * j * kPadRow + d);
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int u = 0; u < 4; ++u)
 #pragma unroll
-            for (int j = 0; j < KJ; ++j) {
-                float v = acc[i][j];
-                v = __builtin_fmaf(a[i].x, c[j].x, v);
-                v = __builtin_fmaf(a[i].y, c[j].y, v);
-                v = __builtin_fmaf(a[i].z, c[j].z, v);
-                v = __builtin_fmaf(a[i].w, c[j].w, v);
-                acc[i][j] = v;
+            for (int i = 0; i < CQ; ++i)
+#pragma unroll
+                for (int j = 0; j < CK; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_4x4x1f32(a[i][u], c[j][u], acc[i][j], 0, 0, 0);
+    }
+    // element r of a lane: query row r and key n of its block
+#pragma unroll
+    for (int i = 0; i < CQ; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int m = m0 + wq + 16 * i + bq + r;
+            if (m >= M) continue;
+            const int last = P + m % s.Qb;
+            float* out = logits + ((int64_t)(b * s.Hq + hk * s.G) * s.Qb + m) * s.cap;
+#pragma unroll
+            for (int j = 0; j < CK; ++j) {
+                const int kb = kb0 + wk + 16 * j + bk + n;
+                if (kb <= last) out[kb] = acc[i][j][r] * scale;
             }
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int m = m0 + tm + 16 * i;
-        if (m >= M) continue;
-        const int qb = m % s.Qb;
-        float* out = logits + ((int64_t)(b * s.Hq + hk * s.G) * s.Qb + m) * s.cap;
-#pragma unroll
-        for (int j = 0; j < KJ; ++j) {
-            const int kb = kb0 + KJ * tn + j;
-            if (kb <= P + qb) out[kb] = acc[i][j] * scale;
         }
-    }
-    if (has_extra && t < 64) {
-        // key KT of the tile for query row t: the same sequential fma chain over d = 0..127
-        // (after the tile: beside the tile's chains, in every wave, it measured slower)
-        const int m = m0 + t;
-        float v = 0.0f;
-        for (int d = 0; d < kD; d += 4) {
-            const float4 a = *reinterpret_cast<const float4*>(qt + t * kPadRow + d);
-            const float4 c = *reinterpret_cast<const float4*>(kt + KT * kPadRow + d);
-            v = __builtin_fmaf(a.x, c.x, v);
-            v = __builtin_fmaf(a.y, c.y, v);
-            v = __builtin_fmaf(a.z, c.z, v);
-            v = __builtin_fmaf(a.w, c.w, v);
-        }
-        const int kb = kb0 + KT;
-        if (m < M && kb <= P + m % s.Qb)
-            logits[((int64_t)(b * s.Hq + hk * s.G) * s.Qb + m) * s.cap + kb] = v * scale;
-    }
 }
 
 // ---------------------------------------------------------------------------------------
@@ -414,10 +401,46 @@ __device__ __forceinline__ bool is_finite_f(float v) {
     return (__float_as_uint(v) & 0x7f800000u) != 0x7f800000u;
 }
 
+// A lane's value from the lane s places up in its row of 16 (s = 1, 2, 4, 8; lanes whose source
+// is outside the row read garbage that no caller uses).
+template <int kShift>
+__device__ __forceinline__ float row_up(float v) {
+    return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x100 + kShift, 0xf, 0xf, true));
+}
+// The value of lane ^ 32 and of lane ^ 16 (v_permlane*_swap), without a trip through LDS.
+__device__ __forceinline__ float lane_xor32(float v) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float((threadIdx.x & 32) ? r[0] : r[1]);
+}
+__device__ __forceinline__ float lane_xor16(float v) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float((threadIdx.x & 16) ? r[0] : r[1]);
+}
+// Row rotations reach every lane of a row of 16 in four steps.
+template <int kRot>
+__device__ __forceinline__ float row_rot(float v) {
+    return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x120 + kRot, 0xf, 0xf, false));
+}
+
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-    return v;
+    v = fmaxf(v, row_rot<8>(v));
+    v = fmaxf(v, row_rot<4>(v));
+    v = fmaxf(v, row_rot<2>(v));
+    v = fmaxf(v, row_rot<1>(v));
+    v = fmaxf(v, lane_xor16(v));
+    return fmaxf(v, lane_xor32(v));
+}
+
+// The softmax sum's tree over 64 partials, part[l] += part[l + s] for s = 32, 16, 8, 4, 2, 1:
+// lane 0's result, in every lane.
+__device__ __forceinline__ float wave_tree_sum(float part) {
+    part = part + lane_xor32(part);  // lanes 0..31 hold part[l] + part[l + 32]
+    part = part + lane_xor16(part);
+    part = part + row_up<8>(part);
+    part = part + row_up<4>(part);
+    part = part + row_up<2>(part);
+    part = part + row_up<1>(part);
+    return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(part)));
 }
 
 __device__ __forceinline__ int wave_sum_int(int v) {
@@ -467,20 +490,46 @@ __device__ __forceinline__ int wave_kth_smallest_id(const int (&id)[S], const bo
     return T;
 }
 
-// The k-th largest key T over the nl (<= 64 S) candidates held S per lane, and the id cut
-// among the candidates equal to T: the (k - #{key > T})-th smallest such id.
-template <int S>
-__device__ __forceinline__ void select_candidates(const uint32_t* cand_key, const int* cand_id, int nl, int lane,
-                                                  int k, uint32_t& T, int& eq_cut) {
-    uint32_t x[S];
-    int id[S];
-    bool eq[S];
+// A lower bound of the k-th largest of the wave's 64 values (k >= 1): their k-th largest upper
+// half, in 16 rounds.  Half the rounds of the exact one, for a few more candidates above it.
+__device__ __forceinline__ uint32_t wave_kth_bound(uint32_t x, int k) {
+    const uint32_t hi = x >> 16;
+    uint32_t T = 0;
 #pragma unroll
-    for (int i = 0; i < S; ++i) {
-        const int j = lane + 64 * i;
-        x[i] = j < nl ? cand_key[j] : 0u;
-        id[i] = j < nl ? cand_id[j] : 0;
+    for (int bit = 15; bit >= 0; --bit) {
+        const uint32_t c = T | (1u << bit);
+        if (__popcll(__ballot(hi >= c)) >= k) T = c;
     }
+    return T << 16;
+}
+
+// select_candidates for nl <= 64 candidates, one per lane: each counts the candidates before it in
+// the order (key desc, id asc); the one with k - 1 of them holds T and the cut.  nl rounds of
+// four instructions against 48 ballot rounds of a search (nl is a few more than k).
+__device__ __forceinline__ void rank_candidates(uint32_t key, int id, int nl, int lane, int k, uint32_t& T,
+                                                int& eq_cut) {
+    const uint64_t mine = (uint64_t)key << 32 | (uint32_t)~id;
+    int before = 0;
+    for (int j0 = 0; j0 < nl; j0 += 4) {  // (lanes past nl hold key 0: before nobody)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const uint64_t other = (uint64_t)__builtin_amdgcn_readlane(key, j0 + u) << 32 |
+                                   (uint32_t)~__builtin_amdgcn_readlane(id, j0 + u);
+            before += other > mine ? 1 : 0;
+        }
+    }
+    const uint64_t who = __ballot(lane < nl && before == k - 1);
+    const int at = __ffsll(static_cast<unsigned long long>(who)) - 1;
+    T = __builtin_amdgcn_readlane(key, at);
+    eq_cut = __builtin_amdgcn_readlane(id, at);
+}
+
+// The k-th largest key T over candidates held S per lane (key 0: none), and the id cut among the
+// candidates equal to T: the (k - #{key > T})-th smallest such id.
+template <int S>
+__device__ __forceinline__ void select_candidates(const uint32_t (&x)[S], const int (&id)[S], int k, uint32_t& T,
+                                                  int& eq_cut) {
+    bool eq[S];
     T = wave_kth_largest<S>(x, k);
     int gt = 0;
 #pragma unroll
@@ -657,9 +706,7 @@ __global__ __launch_bounds__(kSelThreads) void row_select_kernel(SelectParams p)
         if (wave == 0) {
             uint32_t lo = 0;
             if (k <= 64) {
-                const uint32_t m[1] = {max(max(tmax[lane], tmax[lane + 64]),
-                                           max(tmax[lane + 128], tmax[lane + 192]))};
-                lo = wave_kth_largest<1>(m, k);
+                lo = wave_kth_bound(max(max(tmax[lane], tmax[lane + 64]), max(tmax[lane + 128], tmax[lane + 192])), k);
             }
             if (lane == 0) sel_lo = lo;
         }
@@ -683,9 +730,17 @@ __global__ __launch_bounds__(kSelThreads) void row_select_kernel(SelectParams p)
             int eq_cut;
             if (nl <= 64) {
                 // the usual case: one candidate per lane
-                select_candidates<1>(cand_key, cand_id, nl, lane, k, T, eq_cut);
+                rank_candidates(lane < nl ? cand_key[lane] : 0u, lane < nl ? cand_id[lane] : 0, nl, lane, k, T, eq_cut);
             } else if (nl <= kCandCap) {
-                select_candidates<kCandSlots>(cand_key, cand_id, nl, lane, k, T, eq_cut);
+                uint32_t x[kCandSlots];
+                int id[kCandSlots];
+#pragma unroll
+                for (int i = 0; i < kCandSlots; ++i) {
+                    const int j = lane + 64 * i;
+                    x[i] = j < nl ? cand_key[j] : 0u;
+                    id[i] = j < nl ? cand_id[j] : 0;
+                }
+                select_candidates<kCandSlots>(x, id, k, T, eq_cut);
             } else {
                 T = 0;
                 for (int bit = 31; bit >= 0; --bit) {
@@ -760,27 +815,40 @@ __global__ __launch_bounds__(kSelThreads) void row_select_kernel(SelectParams p)
     }
 }
 
+// v / sum, correctly rounded: with y the correctly rounded reciprocal and q = v y, the remainder
+// v - sum q is exact in an fma and q + y (v - sum q) rounds as the quotient (Markstein's division),
+// for sum and v of normal size; four instructions for a divisor that the row shares against ten.
+// The caller sends quotients that may be subnormal, and sums that are not finite, to a division.
+__device__ __forceinline__ float div_by(float v, float sum, float y) {
+    const float q = v * y;
+    return __builtin_fmaf(__builtin_fmaf(-sum, q, v), y, q);
+}
+
 // The same row selection with the row held in registers, for rows of at most 256 * NR
 // blocks: thread t owns blocks kb = t + 256 i (i < NR), which is also lane (kb % 64) of
 // wave (kb / 64) % 4 in mask chunk kb / 64, so the masks come straight from registers.
 //  - one round of global loads for the whole row;
-//  - the softmax sum keeps the order above (wave 0 over the exponentials staged in LDS);
-//  - every wave derives the top-k bound and the final cut itself from the shared lane
-//    maxima and candidate list, which saves the broadcast barriers;
-//  - the row is also staged in LDS for the whole-row search when the candidate list
-//    overflows.
-// Results are bit-identical to row_select_kernel.
+//  - the softmax sum keeps the order above; every wave adds the exponentials staged in LDS
+//    itself, so its result needs no barrier;
+//  - a block's order key is made once (0: not a candidate; a finite float's key is never 0) and
+//    serves the bound, the candidate list and the masks;
+//  - each wave lists its candidates by ballots in its own part of the list, and every wave
+//    derives the top-k bound and the final cut itself;
+//  - a candidate list that overflows falls back to the whole-row search.
+// Results are bit-identical to row_select_kernel.  Bound by the latency of its phases, which is
+// what these choices cut: 512 rows of 2064 blocks, top-k 10, 16.2 -> 12.7 us; 896 rows of up to
+// 2056 17.0 -> 12.7; 256 rows of 1032 9.4 -> 7.1; 128 rows of 128 6.2 -> 4.9.
 template <bool kCompute, int NR>
 __global__ __launch_bounds__(kSelThreads) void row_select_reg_kernel(SelectParams p) {
     extern __shared__ float row[];  // [cap]
     __shared__ float red_f[kSelWaves];
-    __shared__ float red_sum;  // its own slot: the statistics below reuse red_f without a barrier
+    __shared__ float red_m[kSelWaves];  // its own slots: the statistics reuse no array without a barrier
     __shared__ int red_i[kSelWaves];
     __shared__ int red_z[kSelWaves];
+    __shared__ int red_n[kSelWaves];
     __shared__ uint32_t tmax[kSelThreads];
-    __shared__ uint32_t cand_key[kCandCap];
-    __shared__ int cand_id[kCandCap];
-    __shared__ int cand_n;
+    __shared__ uint32_t cand_key[kSelWaves][kCandCap];
+    __shared__ int cand_id[kSelWaves][kCandCap];
     __shared__ uint32_t sel_T;
     __shared__ int sel_cut;
     const Shape& s = p.s;
@@ -791,7 +859,7 @@ __global__ __launch_bounds__(kSelThreads) void row_select_reg_kernel(SelectParam
     const int h = bh - b * s.Hq;
     const int t = threadIdx.x;
     const int lane = t & 63;
-    const int wave = t >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int P = p.pb.p[b];
     const int qabs = P + qb;
     const int n = qabs + 1;
@@ -823,37 +891,36 @@ __global__ __launch_bounds__(kSelThreads) void row_select_reg_kernel(SelectParam
             }
         }
         __syncthreads();
-        if (wave == 0) {
-            // lane l sums kb = l, l + 64, ... in ascending order, then the fixed tree
-            float part = 0.0f;
-            for (int base = 0; base < n; base += 8 * 64) {
-                float e[8];
+        // lane l sums kb = l, l + 64, ... in ascending order (a column past the row adds nothing),
+        // then the fixed tree
+        float part = 0.0f;
+        {
+            float e[4 * NR];
 #pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const int kb = base + lane + 64 * i;
-                    e[i] = kb < n ? row[kb] : 0.0f;
-                }
+            for (int i = 0; i < 4 * NR; ++i) e[i] = row[min(lane + 64 * i, n - 1)];
 #pragma unroll
-                for (int i = 0; i < 8; ++i)
-                    if (base + lane + 64 * i < n) part = part + e[i];
-            }
-#pragma unroll
-            for (int o = 32; o >= 1; o >>= 1) part = part + __shfl_down(part, o, 64);
-            if (lane == 0) red_sum = part;
+            for (int i = 0; i < 4 * NR; ++i) part = lane + 64 * i < n ? part + e[i] : part;
         }
-        __syncthreads();
-        const float sum = red_sum;
+        const float sum = wave_tree_sum(part);
+        const float y = 1.0f / sum;
+        // a weight is 0 or at least e^-80: tiny ones could give subnormal quotients
+        float least = 1.0f;
 #pragma unroll
         for (int i = 0; i < NR; ++i) {
-            const int kb = t + kSelThreads * i;
-            float pv = 0.0f;
-            if (kb < n) {
-                pv = v[i] / sum;
-                row[kb] = pv;
-            }
-            v[i] = pv;
-            if (kb < cap) srow[kb] = pv;
+            if (t + kSelThreads * i >= n) v[i] = 0.0f;
+            least = fminf(least, v[i] != 0.0f ? v[i] : 1.0f);
         }
+        if (sum >= 1.0f && sum < 1e9f && __ballot(least < 1e-25f) == 0) {
+#pragma unroll
+            for (int i = 0; i < NR; ++i) v[i] = div_by(v[i], sum, y);
+        } else {
+#pragma unroll
+            for (int i = 0; i < NR; ++i)
+                if (t + kSelThreads * i < n) v[i] = v[i] / sum;
+        }
+#pragma unroll
+        for (int i = 0; i < NR; ++i)
+            if (t + kSelThreads * i < cap) srow[t + kSelThreads * i] = v[i];
     } else {
         const int64_t off = b * p.ssb + h * p.ssh + qb * p.ssq;
         // unconditional loads of a clamped column (n >= 1), all in flight at once
@@ -869,185 +936,184 @@ __global__ __launch_bounds__(kSelThreads) void row_select_reg_kernel(SelectParam
 #pragma unroll
         for (int i = 0; i < NR; ++i)
             if (t + kSelThreads * i >= n) v[i] = 0.0f;
-#pragma unroll
-        for (int i = 0; i < NR; ++i) {
-            const int kb = t + kSelThreads * i;
-            if (kb < n) row[kb] = v[i];
-        }
     }
 
-    // Row statistics as in row_select_kernel: the zeroed row's max over all Kb columns,
-    // the top-k candidate count and each thread's largest candidate key.
+    // Candidate keys, the top-k candidate count and each thread's largest key, as in
+    // row_select_kernel; under the alpha rule the zeroed row's max over all Kb columns.
     const ca_select_rule& rule = p.rule;
     const int Kb = P + s.Qb;
     const bool all_cols = (rule.flags & CA_RULE_TOPK_ALLCOLS) != 0;
+    const bool use_alpha = (rule.flags & CA_RULE_ALPHA) != 0;
     const int kend = all_cols ? Kb : P;
     const bool use_topk = (rule.flags & CA_RULE_TOPK) && rule.topk > 0 && kend > 0;
-    // candidate value of register i (block kb): the zeroed value over all columns, or a
-    // finite past score
-    auto cand_val = [&](int i, int kb, float& cv) -> bool {
-        if (all_cols) {
-            cv = kb < n ? v[i] : 0.0f;
-            if (!is_finite_f(cv)) cv = 0.0f;
-            return true;
-        }
-        cv = v[i];
-        return is_finite_f(cv);
-    };
-    {
-        float mx = kNegInf;
-        int nc = 0, nz = 0;
+    const int k = rule.topk;
+    uint32_t key[NR];
+    if (use_topk) {
         uint32_t kmax = 0;
+        int nc = 0;
 #pragma unroll
         for (int i = 0; i < NR; ++i) {
             const int kb = t + kSelThreads * i;
-            if (kb < n) {
-                if (is_finite_f(v[i]))
-                    mx = fmaxf(mx, v[i]);
-                else
-                    ++nz;
-            }
-            float cv;
-            if (use_topk && kb < kend && cand_val(i, kb, cv)) {
-                ++nc;
-                kmax = max(kmax, order_key(cv));
-            }
+            const bool fin = is_finite_f(v[i]);
+            // the zeroed value over all columns, or a finite past score
+            const float cv = fin && kb < n ? v[i] : 0.0f;
+            const bool cand = kb < kend && (all_cols || fin);
+            key[i] = cand ? order_key(cv) : 0u;
+            kmax = max(kmax, key[i]);
+            nc += __popcll(__ballot(cand));
+        }
+        tmax[t] = kmax;
+        if (lane == 0) red_i[wave] = nc;
+    }
+    if (use_alpha) {
+        float mx = kNegInf;
+        uint64_t bad = 0;
+#pragma unroll
+        for (int i = 0; i < NR; ++i) {
+            const bool in = t + kSelThreads * i < n;
+            const bool fin = is_finite_f(v[i]);
+            if (in && fin) mx = fmaxf(mx, v[i]);
+            bad |= __ballot(in && !fin);
         }
         mx = wave_max(mx);
-        nc = wave_sum_int(nc);
-        nz = wave_sum_int(nz);
-        tmax[t] = kmax;
         if (lane == 0) {
-            red_f[wave] = mx;
-            red_i[wave] = nc;
-            red_z[wave] = nz;
+            red_m[wave] = mx;
+            red_z[wave] = bad != 0;
         }
-        if (t == 0) cand_n = 0;
     }
     __syncthreads();
-    float rowmax = fmaxf(fmaxf(red_f[0], red_f[1]), fmaxf(red_f[2], red_f[3]));
-    if (n < Kb || red_z[0] + red_z[1] + red_z[2] + red_z[3] > 0) rowmax = fmaxf(rowmax, 0.0f);
-    const int ncand = red_i[0] + red_i[1] + red_i[2] + red_i[3];
-    const float alpha_cut = rule.alpha * rowmax;
-    const bool take_all = use_topk && rule.topk >= ncand;
-    const bool cut = use_topk && !take_all;
-    const int k = rule.topk;
-
+    float alpha_cut = 0.0f;
+    if (use_alpha) {
+        float rowmax = fmaxf(fmaxf(red_m[0], red_m[1]), fmaxf(red_m[2], red_m[3]));
+        if (n < Kb || (red_z[0] | red_z[1] | red_z[2] | red_z[3])) rowmax = fmaxf(rowmax, 0.0f);
+        alpha_cut = rule.alpha * rowmax;
+    }
+    bool take_all = false;
     uint32_t T = 0u;
     int eq_cut = -1;
-    if (cut) {
-        // every wave computes the same lower bound from the 64 lane maxima
-        uint32_t lo = 0;
-        if (k <= 64) {
-            const uint32_t m1[1] = {max(max(tmax[lane], tmax[lane + 64]), max(tmax[lane + 128], tmax[lane + 192]))};
-            lo = wave_kth_largest<1>(m1, k);
-        }
+    if (use_topk) {
+        take_all = k >= red_i[0] + red_i[1] + red_i[2] + red_i[3];
+        if (!take_all) {
+            // every wave computes the same lower bound from the 64 lane maxima (1: any candidate)
+            uint32_t lo = 1;
+            if (k <= 64)
+                lo = max(1u, wave_kth_bound(
+                                 max(max(tmax[lane], tmax[lane + 64]), max(tmax[lane + 128], tmax[lane + 192])), k));
+            int mine = 0;
+            const uint64_t lt_mask = (1ull << lane) - 1ull;
 #pragma unroll
-        for (int i = 0; i < NR; ++i) {
-            const int kb = t + kSelThreads * i;
-            float cv;
-            if (kb < kend && cand_val(i, kb, cv)) {
-                const uint32_t key = order_key(cv);
-                if (key >= lo) {
-                    const int slot = atomicAdd(&cand_n, 1);
-                    if (slot < kCandCap) {
-                        cand_key[slot] = key;
-                        cand_id[slot] = kb;
+            for (int i = 0; i < NR; ++i) {
+                const bool c = key[i] >= lo;
+                const uint64_t bal = __ballot(c);
+                if (bal != 0) {
+                    const int slot = mine + __popcll(bal & lt_mask);
+                    if (c && slot < kCandCap) {
+                        cand_key[wave][slot] = key[i];
+                        cand_id[wave][slot] = t + kSelThreads * i;
                     }
+                    mine += __popcll(bal);
                 }
             }
-        }
-        __syncthreads();
-        const int nl = cand_n;
-        if (nl <= 64) {
-            select_candidates<1>(cand_key, cand_id, nl, lane, k, T, eq_cut);  // every wave, same result
-        } else if (nl <= kCandCap) {
-            select_candidates<kCandSlots>(cand_key, cand_id, nl, lane, k, T, eq_cut);
-        } else {
-            // heavy ties or k > 64: wave 0 searches the staged row, as row_select_kernel does
-            if (wave == 0) {
-                auto row_val = [&](int kb, float& cv) -> bool {
-                    if (all_cols) {
-                        cv = kb < n ? row[kb] : 0.0f;
-                        if (!is_finite_f(cv)) cv = 0.0f;
-                        return true;
+            if (lane == 0) red_n[wave] = mine;
+            __syncthreads();
+            const int n0 = red_n[0], n1 = n0 + red_n[1], n2 = n1 + red_n[2], nl = n2 + red_n[3];
+            auto cand = [&](int j, uint32_t& ck, int& ci) {  // entry j of the four waves' lists in a row
+                const int wv = (j >= n0) + (j >= n1) + (j >= n2);
+                const int at = j - (wv == 0 ? 0 : wv == 1 ? n0 : wv == 2 ? n1 : n2);
+                ck = j < nl ? cand_key[wv][at] : 0u;
+                ci = j < nl ? cand_id[wv][at] : 0;
+            };
+            if (nl <= 64) {
+                uint32_t ck;
+                int ci;
+                cand(lane, ck, ci);
+                rank_candidates(ck, ci, nl, lane, k, T, eq_cut);
+            } else if (nl <= kCandCap) {
+                uint32_t ck[kCandSlots];
+                int ci[kCandSlots];
+#pragma unroll
+                for (int i = 0; i < kCandSlots; ++i) cand(lane + 64 * i, ck[i], ci[i]);
+                select_candidates<kCandSlots>(ck, ci, k, T, eq_cut);
+            } else {
+                // heavy ties or k > 64: the row goes to LDS and wave 0 searches it, as
+                // row_select_kernel does (the exponentials there were last read before the barriers above)
+#pragma unroll
+                for (int i = 0; i < NR; ++i)
+                    if (t + kSelThreads * i < n) row[t + kSelThreads * i] = v[i];
+                __syncthreads();
+                if (wave == 0) {
+                    auto row_val = [&](int kb, float& cv) -> bool {
+                        if (all_cols) {
+                            cv = kb < n ? row[kb] : 0.0f;
+                            if (!is_finite_f(cv)) cv = 0.0f;
+                            return true;
+                        }
+                        cv = row[kb];
+                        return is_finite_f(cv);
+                    };
+                    uint32_t Tw = 0;
+                    for (int bit = 31; bit >= 0; --bit) {
+                        const uint32_t c = Tw | (1u << bit);
+                        int cnt = 0;
+                        for (int kb = lane; kb < kend; kb += 64) {
+                            float cv;
+                            cnt += (row_val(kb, cv) && order_key(cv) >= c) ? 1 : 0;
+                        }
+                        if (wave_sum_int(cnt) >= k) Tw = c;
                     }
-                    cv = row[kb];
-                    return is_finite_f(cv);
-                };
-                uint32_t Tw = 0;
-                for (int bit = 31; bit >= 0; --bit) {
-                    const uint32_t c = Tw | (1u << bit);
-                    int cnt = 0;
+                    int gt = 0;
                     for (int kb = lane; kb < kend; kb += 64) {
                         float cv;
-                        cnt += (row_val(kb, cv) && order_key(cv) >= c) ? 1 : 0;
+                        gt += (row_val(kb, cv) && order_key(cv) > Tw) ? 1 : 0;
                     }
-                    if (wave_sum_int(cnt) >= k) Tw = c;
-                }
-                int gt = 0;
-                for (int kb = lane; kb < kend; kb += 64) {
-                    float cv;
-                    gt += (row_val(kb, cv) && order_key(cv) > Tw) ? 1 : 0;
-                }
-                const int krem = k - wave_sum_int(gt);
-                const uint64_t lt_mask = (1ull << lane) - 1ull;
-                int seen = 0;
-                int cutw = kend;
-                for (int base = 0; base < kend; base += 64) {
-                    const int kb = base + lane;
-                    float cv = 0.0f;
-                    const bool e = kb < kend && row_val(kb, cv) && order_key(cv) == Tw;
-                    const uint64_t bal = __ballot(e);
-                    const int cnt = __popcll(bal);
-                    if (seen + cnt >= krem) {
-                        const uint64_t who = __ballot(e && seen + __popcll(bal & lt_mask) == krem - 1);
-                        cutw = base + __ffsll(static_cast<unsigned long long>(who)) - 1;
-                        break;
+                    const int krem = k - wave_sum_int(gt);
+                    int seen = 0;
+                    int cutw = kend;
+                    for (int base = 0; base < kend; base += 64) {
+                        const int kb = base + lane;
+                        float cv = 0.0f;
+                        const bool e = kb < kend && row_val(kb, cv) && order_key(cv) == Tw;
+                        const uint64_t bal = __ballot(e);
+                        const int cnt = __popcll(bal);
+                        if (seen + cnt >= krem) {
+                            const uint64_t who = __ballot(e && seen + __popcll(bal & lt_mask) == krem - 1);
+                            cutw = base + __ffsll(static_cast<unsigned long long>(who)) - 1;
+                            break;
+                        }
+                        seen += cnt;
                     }
-                    seen += cnt;
+                    if (lane == 0) {
+                        sel_T = Tw;
+                        sel_cut = cutw;
+                    }
                 }
-                if (lane == 0) {
-                    sel_T = Tw;
-                    sel_cut = cutw;
-                }
+                __syncthreads();
+                T = sel_T;
+                eq_cut = sel_cut;
             }
-            __syncthreads();
-            T = sel_T;
-            eq_cut = sel_cut;
         }
     }
 
     // masks: register i of this thread is lane `lane` of chunk c = wave + 4 i
     uint32_t* out = p.rowmask + (int64_t)rid * s.words;
     const int chunks = (s.words + 1) / 2;
+    const bool use_thr = (rule.flags & CA_RULE_THRESHOLD) != 0;
+    const int w0 = qabs - max(rule.window_blocks, 0) + 1;  // the window: ids from w0 on
+    const int local = max(rule.local_blocks, 0);           // the local past blocks: [l0, l0 + local)
+    const int l0 = P - local;
 #pragma unroll
     for (int i = 0; i < NR; ++i) {
         const int c = wave + kSelWaves * i;
         if (c >= chunks) break;
         const int kb = c * 64 + lane;
-        bool keep = false;
-        if (kb < n) {
-            const float x = v[i];
-            const bool fin = is_finite_f(x);
-            if ((rule.flags & CA_RULE_ALPHA) && fin && x >= alpha_cut) keep = true;
-            if ((rule.flags & CA_RULE_THRESHOLD) && x > rule.threshold) keep = true;
-            if (kb < rule.sink_blocks) keep = true;
-            if (qabs - kb < rule.window_blocks) keep = true;
-            if (kb < P && kb >= P - rule.local_blocks) keep = true;
-            float cv;
-            if (use_topk && kb < kend && cand_val(i, kb, cv)) {
-                if (take_all) {
-                    keep = true;
-                } else {
-                    const uint32_t key = order_key(cv);
-                    if (key > T || (key == T && kb <= eq_cut)) keep = true;
-                }
-            }
-        }
-        const uint64_t bal = __ballot(keep);
-        if (lane == 0) out[2 * c] = static_cast<uint32_t>(bal);
-        if (lane == 1 && 2 * c + 1 < s.words) out[2 * c + 1] = static_cast<uint32_t>(bal >> 32);
+        uint64_t bits = __ballot(kb < rule.sink_blocks || kb >= w0 || (unsigned)(kb - l0) < (unsigned)local);
+        // top-k: above the cut key, or at it up to the last kept id (every candidate: key > 0)
+        if (use_topk) bits |= __ballot(key[i] > T || (key[i] == T && kb <= eq_cut));
+        if (use_alpha) bits |= __ballot(is_finite_f(v[i]) && v[i] >= alpha_cut);
+        if (use_thr) bits |= __ballot(v[i] > rule.threshold);
+        bits &= __ballot(kb < n);
+        if (lane == 0) out[2 * c] = static_cast<uint32_t>(bits);
+        if (lane == 1 && 2 * c + 1 < s.words) out[2 * c + 1] = static_cast<uint32_t>(bits >> 32);
     }
 }
 
@@ -1306,21 +1372,18 @@ hipError_t launch_score_select(const Shape& s, const float* qhat, const float* k
     if (compute) {
         int max_nkb = 0;
         for (int b = 0; b < s.B; ++b) max_nkb = max(max_nkb, pb.p[b] + s.Qb);
-        constexpr int kKT = 32;
-        const int rows_z = s.B * s.Hkv * ((s.G * s.Qb + 63) / 64);
-        int tiles = (max_nkb + kKT - 1) / kKT;
-        int extra = 0;
-        // two workgroups on each of the 256 CUs: when the 32-key tiles overflow that by a few
-        // tiles per row, fit the row into kLogitsGridSlots / rows tiles, the first of them
-        // holding 33 keys (at most one more key per tile)
-        const int fit = kLogitsGridSlots / rows_z;
-        if (tiles * rows_z > kLogitsGridSlots && fit >= 1 && fit < tiles && max_nkb <= fit * (kKT + 1)) {
-            tiles = fit;
-            extra = max_nkb - fit * kKT;
-        }
-        dim3 grid(tiles, s.B * s.Hkv, (s.G * s.Qb + 63) / 64);
-        hipLaunchKernelGGL(block_logits_kernel<kKT>, grid, dim3(256), 0, stream, s, qhat, khat, scale, pb, scores,
-                           extra);
+        // query vectors of a KV group per workgroup: 16, 32 or 64
+        const int M = s.G * s.Qb;
+        auto launch = [&](auto kernel, int nq) {
+            dim3 grid((max_nkb + kLogitsKeys - 1) / kLogitsKeys, s.B * s.Hkv, (M + 16 * nq - 1) / (16 * nq));
+            hipLaunchKernelGGL(kernel, grid, dim3(64 * nq), 0, stream, s, qhat, khat, scale, pb, scores);
+        };
+        if (M <= 16)
+            launch(block_logits_kernel<1>, 1);
+        else if (M <= 32)
+            launch(block_logits_kernel<2>, 2);
+        else
+            launch(block_logits_kernel<4>, 4);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
@@ -1339,14 +1402,22 @@ hipError_t launch_score_select(const Shape& s, const float* qhat, const float* k
     dim3 grid(s.B * s.Hq * s.Qb);
     // rows of up to 16 * 256 blocks (262144 tokens) in registers, longer ones through LDS
     auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kSelThreads), lds, stream, p); };
-    if (s.cap <= 4 * kSelThreads)
-        compute ? launch(row_select_reg_kernel<true, 4>) : launch(row_select_reg_kernel<false, 4>);
-    else if (s.cap <= 8 * kSelThreads)
-        compute ? launch(row_select_reg_kernel<true, 8>) : launch(row_select_reg_kernel<false, 8>);
+    auto pick = [&](auto nr) {
+        constexpr int NR = decltype(nr)::value;
+        compute ? launch(row_select_reg_kernel<true, NR>) : launch(row_select_reg_kernel<false, NR>);
+    };
+    if (s.cap <= 2 * kSelThreads)
+        pick(std::integral_constant<int, 2>{});
+    else if (s.cap <= 4 * kSelThreads)
+        pick(std::integral_constant<int, 4>{});
+    else if (s.cap <= 6 * kSelThreads)
+        pick(std::integral_constant<int, 6>{});
+    else if (s.cap <= 9 * kSelThreads)
+        pick(std::integral_constant<int, 9>{});
     else if (s.cap <= 12 * kSelThreads)
-        compute ? launch(row_select_reg_kernel<true, 12>) : launch(row_select_reg_kernel<false, 12>);
+        pick(std::integral_constant<int, 12>{});
     else if (s.cap <= 16 * kSelThreads)
-        compute ? launch(row_select_reg_kernel<true, 16>) : launch(row_select_reg_kernel<false, 16>);
+        pick(std::integral_constant<int, 16>{});
     else
         compute ? launch(row_select_kernel<true>) : launch(row_select_kernel<false>);
     return hipGetLastError();
