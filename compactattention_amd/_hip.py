@@ -49,6 +49,8 @@ EXPORTED = (
     "ca_score_token_mass",
     "ca_select_scores",
     "ca_union_compact",
+    "ca_union_compact_pairs",
+    "ca_append_tokens",
     "ca_compact_keep_kv",
     "ca_dense_table",
     "ca_table_to_csr",
@@ -59,6 +61,7 @@ EXPORTED = (
     "ca_attn_decode",
     "ca_attn_decode_workspace_size",
     "ca_rope_apply",
+    "ca_rope_qk",
     "ca_rmsnorm",
     "ca_swiglu",
 )
@@ -140,6 +143,9 @@ _SIGNATURES = {
     "ca_score_token_mass": (ctypes.c_int, [_P(Dims), _P(SeqLayout), _vp, _i64, _i32, _f32, _vp, _vp, _vp]),
     "ca_select_scores": (ctypes.c_int, [_P(Dims), _vp, _i32, _i64, _i64, _i64, _P(SelectRule), _vp, _vp, _vp]),
     "ca_union_compact": (ctypes.c_int, [_P(Dims), _vp, _i32, _vp, _vp, _vp, _vp, _i64, _vp, _vp]),
+    "ca_union_compact_pairs": (ctypes.c_int, [_P(Dims), _vp, _i32, _vp, _vp, _i64, _vp, _i32, _vp, _i64, _i32, _vp,
+                                              _vp]),
+    "ca_append_tokens": (ctypes.c_int, [_P(Dims), _P(SeqLayout), _P(SeqLayout), _P(KvLayout), _P(KvLayout), _i64, _vp]),
     "ca_compact_keep_kv": (ctypes.c_int, [_P(Dims), _vp, _vp, _vp, _i64, _vp, _vp]),
     "ca_dense_table": (ctypes.c_int, [_P(Dims), _vp, _vp, _i64, _vp, _vp]),
     "ca_table_to_csr": (ctypes.c_int, [_P(Dims), _vp, _i64, _vp, _vp, _vp, _i64, _vp, _vp]),
@@ -153,6 +159,8 @@ _SIGNATURES = {
                                       _P(SeqLayout), _vp, _i32, _vp, _i64, _vp]),
     "ca_attn_decode_workspace_size": (ctypes.c_int64, [_P(Dims), _vp, _i32]),
     "ca_rope_apply": (ctypes.c_int, [_P(SeqLayout), _P(SeqLayout), _i32, _i32, _i32, _vp, _vp, _vp]),
+    "ca_rope_qk": (ctypes.c_int, [_P(SeqLayout), _P(SeqLayout), _i32, _P(SeqLayout), _P(SeqLayout), _i32, _i32, _i32,
+                                  _vp, _vp, _vp]),
     "ca_rmsnorm": (ctypes.c_int, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _i64, _i64, _i32, _f32, _vp]),
     "ca_swiglu": (ctypes.c_int, [_vp, _i64, _vp, _i64, _vp, _i64, _i64, _i32, _vp]),
 }

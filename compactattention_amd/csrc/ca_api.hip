@@ -468,6 +468,59 @@ int ca_union_compact(const ca_dims* dims, const uint32_t* rowmask, int32_t last_
     return ok();
 }
 
+int ca_union_compact_pairs(const ca_dims* dims, const uint32_t* rowmask, int32_t last_n_block,
+                           const int32_t* past_blocks_host, int32_t* table, int64_t table_stride, int32_t* counts,
+                           int32_t key_pages, int32_t* pages, int64_t pages_stride, int32_t page_cap,
+                           int32_t* page_counts, void* stream) {
+    ca::Shape s;
+    ca::PastBlocks pb;
+    int max_nkb = 0, rc;
+    if ((rc = check_dims(dims, past_blocks_host, &s, &pb, &max_nkb)) != CA_OK) return rc;
+    if (rowmask == nullptr || table == nullptr || counts == nullptr || pages == nullptr || page_counts == nullptr)
+        return fail(CA_ERR_INVALID, "rowmask, table, counts, pages and page_counts are required");
+    if (table_stride < s.cap) return fail(CA_ERR_INVALID, "table_stride=%lld < kv_cap=%d", (long long)table_stride, s.cap);
+    for (int b = 0; b < s.B; ++b)
+        if (((int64_t)key_pages + 1) / 2 != (int64_t)pb.p[b] + s.Qb)
+            return fail(CA_ERR_INVALID, "key_pages=%d do not end in request %d's last of %d blocks", key_pages, b,
+                        pb.p[b] + s.Qb);
+    if (page_cap < key_pages || pages_stride < page_cap)
+        return fail(CA_ERR_INVALID, "rows of %d pages (stride %lld) do not hold key_pages=%d", page_cap,
+                    (long long)pages_stride, key_pages);
+    if (ca::union_lds_bytes(s) > kMaxLds) return fail(CA_ERR_LIMIT, "kv_cap too large");
+    hipError_t e = ca::launch_union_compact_pairs(s, rowmask, last_n_block, pb, table, table_stride, counts, key_pages,
+                                                  pages, pages_stride, page_cap, page_counts,
+                                                  static_cast<hipStream_t>(stream));
+    if (e != hipSuccess) return hip_fail(e, "union_compact_pairs launch");
+    return ok();
+}
+
+int ca_append_tokens(const ca_dims* dims, const ca_seq_layout* k_new, const ca_seq_layout* v_new,
+                     const ca_kv_layout* k_cache, const ca_kv_layout* v_cache, int64_t start, void* stream) {
+    if (dims == nullptr) return fail(CA_ERR_INVALID, "dims is NULL");
+    if (dims->batch < 1 || dims->q_len < 1 || dims->num_kv_heads < 1)
+        return fail(CA_ERR_INVALID, "batch=%d, q_len=%d and num_kv_heads=%d must be positive", dims->batch, dims->q_len,
+                    dims->num_kv_heads);
+    if (dims->kv_cap < 1 || (int64_t)dims->kv_cap * CA_BLOCK > (int64_t)1 << 30)
+        return fail(dims->kv_cap < 1 ? CA_ERR_INVALID : CA_ERR_LIMIT, "kv_cap=%d blocks outside [1, 2^24]", dims->kv_cap);
+    if (start < 0 || start + dims->q_len > (int64_t)dims->kv_cap * CA_BLOCK)
+        return fail(CA_ERR_INVALID, "tokens [%lld, %lld) outside a cache of %d blocks", (long long)start,
+                    (long long)(start + dims->q_len), dims->kv_cap);
+    if ((int64_t)dims->batch * dims->num_kv_heads * dims->q_len >= (int64_t)1 << 32)
+        return fail(CA_ERR_LIMIT, "too many rows");
+    const int blocks = static_cast<int>((start + dims->q_len + CA_BLOCK - 1) / CA_BLOCK);
+    ca::SeqAddr kn, vn;
+    ca::KvAddr kc, vc;
+    int rc;
+    if ((rc = check_seq(k_new, "k_new", &kn)) != CA_OK) return rc;
+    if ((rc = check_seq(v_new, "v_new", &vn)) != CA_OK) return rc;
+    if ((rc = check_kv(k_cache, "k_cache", blocks, &kc)) != CA_OK) return rc;
+    if ((rc = check_kv(v_cache, "v_cache", blocks, &vc)) != CA_OK) return rc;
+    hipError_t e = ca::launch_append_tokens(dims->batch, dims->q_len, dims->num_kv_heads, kn, vn, kc, vc, start,
+                                            static_cast<hipStream_t>(stream));
+    if (e != hipSuccess) return hip_fail(e, "append_tokens launch");
+    return ok();
+}
+
 int ca_compact_keep_kv(const ca_dims* dims, const uint8_t* keep_kv, const int32_t* past_blocks_host,
                        int32_t* table, int64_t table_stride, int32_t* counts, void* stream) {
     ca::Shape s;
@@ -659,20 +712,40 @@ int ca_attn_decode(const ca_dims* dims, const ca_seq_layout* q, const ca_kv_layo
 // ---------------------------------------------------------------------------------------
 // Model plumbing: fused element-wise kernels of the Llama integration.
 
-int ca_rope_apply(const ca_seq_layout* x, const ca_seq_layout* y, int32_t batch, int32_t len, int32_t heads,
-                  const float* cos, const float* sin, void* stream) {
-    ca::SeqAddr xa, ya;
+namespace {
+int rope(const ca_seq_layout* x, const ca_seq_layout* y, int32_t heads, const ca_seq_layout* x2, const ca_seq_layout* y2,
+         int32_t heads2, int32_t batch, int32_t len, const float* cos, const float* sin, void* stream) {
+    ca::SeqAddr xa, ya, xb, yb;
     int rc;
     if ((rc = check_seq(x, "x", &xa)) != CA_OK) return rc;
     if ((rc = check_seq(y, "y", &ya)) != CA_OK) return rc;
+    const bool two = heads2 > 0;
+    if (two) {
+        if ((rc = check_seq(x2, "k", &xb)) != CA_OK) return rc;
+        if ((rc = check_seq(y2, "k_out", &yb)) != CA_OK) return rc;
+    }
     if (batch < 1 || len < 1 || heads < 1) return fail(CA_ERR_INVALID, "batch, len and heads must be positive");
-    if ((int64_t)batch * len >= ((int64_t)1 << 31) || heads > 65535)
+    if ((int64_t)batch * len >= ((int64_t)1 << 31) || heads > 65535 || heads2 > 65535)
         return fail(CA_ERR_LIMIT, "batch * len must be below 2^31 and heads at most 65535");
     if (cos == nullptr || sin == nullptr) return fail(CA_ERR_INVALID, "cos and sin are required");
     if (!aligned16(cos) || !aligned16(sin)) return fail(CA_ERR_INVALID, "cos and sin must be 16-byte aligned");
-    hipError_t e = ca::launch_rope(xa, ya, cos, sin, batch, len, heads, static_cast<hipStream_t>(stream));
+    hipError_t e = ca::launch_rope(xa, ya, heads, two ? &xb : nullptr, two ? &yb : nullptr, heads2, cos, sin, batch, len,
+                                   static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return hip_fail(e, "rope launch");
     return ok();
+}
+}  // namespace
+
+int ca_rope_apply(const ca_seq_layout* x, const ca_seq_layout* y, int32_t batch, int32_t len, int32_t heads,
+                  const float* cos, const float* sin, void* stream) {
+    return rope(x, y, heads, nullptr, nullptr, 0, batch, len, cos, sin, stream);
+}
+
+int ca_rope_qk(const ca_seq_layout* q, const ca_seq_layout* q_out, int32_t q_heads, const ca_seq_layout* k,
+               const ca_seq_layout* k_out, int32_t k_heads, int32_t batch, int32_t len, const float* cos,
+               const float* sin, void* stream) {
+    if (k_heads < 1) return fail(CA_ERR_INVALID, "k_heads must be positive");
+    return rope(q, q_out, q_heads, k, k_out, k_heads, batch, len, cos, sin, stream);
 }
 
 int ca_rmsnorm(const uint16_t* x, int64_t x_stride, const uint16_t* residual, int64_t r_stride, uint16_t* sum_out,

@@ -82,6 +82,15 @@ hipError_t launch_union_compact(const Shape& s, const uint32_t* rowmask, int las
                                 const uint8_t* keep_kv_in, const PastBlocks& pb, uint8_t* keep_block,
                                 uint8_t* keep_kv, int32_t* table, int64_t table_stride,
                                 int32_t* counts, bool dense, hipStream_t stream);
+// The same over 128-token blocks, with the tables in 64-token pages too: key_pages per row exist,
+// rows of pages hold page_cap entries
+hipError_t launch_union_compact_pairs(const Shape& s, const uint32_t* rowmask, int last_n_block, const PastBlocks& pb,
+                                      int32_t* table, int64_t table_stride, int32_t* counts, int key_pages,
+                                      int32_t* pages, int64_t pages_stride, int page_cap, int32_t* page_counts,
+                                      hipStream_t stream);
+// Decode append: L tokens per request at position start of the cache
+hipError_t launch_append_tokens(int B, int L, int Hkv, const SeqAddr& k_new, const SeqAddr& v_new,
+                                const KvAddr& k_cache, const KvAddr& v_cache, int64_t start, hipStream_t stream);
 
 struct AttnArgs {
     Shape s;
@@ -136,8 +145,9 @@ int64_t attn_workspace_bytes(const Shape& s, int num_splits);
 hipError_t launch_attn(const AttnArgs& a, hipStream_t stream);
 
 // model plumbing (ca_model.hip)
-hipError_t launch_rope(const SeqAddr& x, const SeqAddr& y, const float* cos, const float* sin, int B, int L, int H,
-                       hipStream_t stream);
+// x2 / y2 (nullable): a second tensor of H2 heads over the same tokens
+hipError_t launch_rope(const SeqAddr& x, const SeqAddr& y, int H, const SeqAddr* x2, const SeqAddr* y2, int H2,
+                       const float* cos, const float* sin, int B, int L, hipStream_t stream);
 hipError_t launch_rmsnorm(const uint16_t* x, int64_t x_stride, const uint16_t* r, int64_t r_stride, uint16_t* s,
                           int64_t s_stride, const uint16_t* w, uint16_t* y, int64_t y_stride, int64_t rows, int n,
                           float eps, hipStream_t stream);

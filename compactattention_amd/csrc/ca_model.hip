@@ -24,27 +24,36 @@ typedef uint16_t u16x8_t __attribute__((ext_vector_type(8)));
 // One thread per 8 elements of a head row: lanes 0-7 hold d = 0..63 (their rotate partner
 // d + 64 is read alongside), lanes 8-15 hold d = 64..127.  blockIdx.x is the token row
 // (b * L + t), so a workgroup covers 16 heads of one token and the thread's head and chunk
-// come from its index without divisions.
-struct RopeParams {
+// come from its index without divisions.  blockIdx.y runs over the head groups of q, then over
+// those of k when both go in one launch.
+struct RopeSide {
     const uint16_t* x;
     int64_t xsb, xst, xsh;
     uint16_t* y;
     int64_t ysb, yst, ysh;
+    int H;
+};
+struct RopeParams {
+    RopeSide side[2];
+    int groups0;       // 16-head groups of side 0
     const float* cos;  // [L, 128] rows for the L positions, row stride 128
     const float* sin;
-    int B, L, H;
+    int L;
 };
 
+template <bool kTwo>
 __global__ __launch_bounds__(256) void rope_kernel(RopeParams p) {
     const int bt = blockIdx.x;
-    const int idx = blockIdx.y * 256 + threadIdx.x;
+    const bool second = kTwo && (int)blockIdx.y >= p.groups0;
+    const RopeSide& sd = p.side[second ? 1 : 0];
+    const int idx = (blockIdx.y - (second ? p.groups0 : 0)) * 256 + threadIdx.x;
     const int h = idx >> 4;
-    if (h >= p.H) return;
+    if (h >= sd.H) return;
     const int c = idx & 15;  // 8-element chunk of the 128-wide row
     const int b = bt / p.L;
     const int t = bt - b * p.L;
-    const uint16_t* xr = p.x + b * p.xsb + (int64_t)t * p.xst + (int64_t)h * p.xsh;
-    uint16_t* yr = p.y + b * p.ysb + (int64_t)t * p.yst + (int64_t)h * p.ysh;
+    const uint16_t* xr = sd.x + b * sd.xsb + (int64_t)t * sd.xst + (int64_t)h * sd.xsh;
+    uint16_t* yr = sd.y + b * sd.ysb + (int64_t)t * sd.yst + (int64_t)h * sd.ysh;
     const int d0 = 8 * c;
     const int dp = d0 < 64 ? d0 + 64 : d0 - 64;  // rotate_half partner
     const u16x8_t xv = *reinterpret_cast<const u16x8_t*>(xr + d0);
@@ -176,24 +185,24 @@ __global__ __launch_bounds__(256) void swiglu_kernel(SwigluParams p) {
 
 }  // namespace
 
-hipError_t launch_rope(const SeqAddr& x, const SeqAddr& y, const float* cos, const float* sin, int B, int L, int H,
-                       hipStream_t stream) {
+hipError_t launch_rope(const SeqAddr& x, const SeqAddr& y, int H, const SeqAddr* x2, const SeqAddr* y2, int H2,
+                       const float* cos, const float* sin, int B, int L, hipStream_t stream) {
     RopeParams p;
-    p.x = x.data;
-    p.xsb = x.sb;
-    p.xst = x.st;
-    p.xsh = x.sh;
-    p.y = y.data;
-    p.ysb = y.sb;
-    p.yst = y.st;
-    p.ysh = y.sh;
+    auto side = [](const SeqAddr& a, const SeqAddr& o, int heads) {
+        return RopeSide{a.data, a.sb, a.st, a.sh, o.data, o.sb, o.st, o.sh, heads};
+    };
+    p.side[0] = side(x, y, H);
+    p.side[1] = x2 != nullptr ? side(*x2, *y2, H2) : RopeSide{};
+    p.groups0 = (H * 16 + 255) / 256;
     p.cos = cos;
     p.sin = sin;
-    p.B = B;
     p.L = L;
-    p.H = H;
-    hipLaunchKernelGGL(rope_kernel, dim3(static_cast<unsigned>((int64_t)B * L), static_cast<unsigned>((H * 16 + 255) / 256)),
-                       dim3(256), 0, stream, p);
+    const int groups1 = x2 != nullptr ? (H2 * 16 + 255) / 256 : 0;
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((int64_t)B * L), static_cast<unsigned>(p.groups0 + groups1)),
+                           dim3(256), 0, stream, p);
+    };
+    groups1 > 0 ? launch(rope_kernel<true>) : launch(rope_kernel<false>);
     return hipGetLastError();
 }
 

@@ -1118,7 +1118,9 @@ __global__ __launch_bounds__(kSelThreads) void row_select_reg_kernel(SelectParam
 }
 
 // ---------------------------------------------------------------------------------------
-// Block-Union + compaction, one (request, KV head) row per workgroup of 256 threads.
+// Block-Union + compaction, one (request, KV head) row per workgroup of 256 threads.  With 128-token
+// blocks the same launch writes the table in 64-token pages, which the attention reads (fifteen
+// element-wise launches before: the operator entry, 549 tokens over 16384, 188 -> 93 us).
 struct UnionParams {
     Shape s;
     const uint32_t* rowmask;  // per-row masks (mode 0)
@@ -1131,6 +1133,12 @@ struct UnionParams {
     int32_t* table;
     int64_t table_stride;
     int32_t* counts;
+    // Blocks that are pairs of 64-token pages: the table in page ids beside the one in block ids
+    int32_t* pages;  // null: no pairs
+    int64_t pages_stride;
+    int32_t* page_counts;
+    int key_pages;  // pages that each row has
+    int page_cap;   // entries of a row of pages
 };
 
 __device__ __forceinline__ uint32_t range_bits(int w, int lo, int hi) {
@@ -1217,12 +1225,23 @@ __global__ __launch_bounds__(256) void union_compact_kernel(UnionParams p) {
     for (int w = w0; w < w1; ++w) {
         uint32_t bits = kvw[w];
         while (bits) {
-            const int i = __ffs(bits) - 1;
-            tab[pos++] = 32 * w + i;
+            const int id = 32 * w + __ffs(bits) - 1;
+            if (p.pages) {
+                // pages 2 id and 2 id + 1; the row's last block, which closes every row, may have one
+                int32_t* pg = p.pages + (int64_t)row * p.pages_stride + 2 * pos;
+                pg[0] = 2 * id;
+                if (2 * id + 1 < p.key_pages) pg[1] = 2 * id + 1;
+            }
+            tab[pos++] = id;
             bits &= bits - 1u;
         }
     }
     for (int i = total + t; i < s.cap; i += 256) tab[i] = -1;
+    if (p.pages) {
+        const int n = 2 * total - (p.key_pages & 1);
+        for (int i = n + t; i < p.page_cap; i += 256) p.pages[(int64_t)row * p.pages_stride + i] = -1;
+        if (t == 0) p.page_counts[row] = n;
+    }
     if (t == 0) p.counts[row] = total;
 }
 
@@ -1317,6 +1336,33 @@ __global__ __launch_bounds__(256) void pair_summaries_kernel(const float* src, i
         out.w = (c0 * m0.w + c1 * m1.w) / n;
     }
     *reinterpret_cast<float4*>(dst + (row * dst_stride + j) * kD + 4 * q) = out;
+}
+
+// Decode append: token t of request b, KV head h goes to position start + t of its row, through the
+// page table when there is one.  One thread per 16 bytes of K and of V.  Bound by its launch: it
+// stands for the page indices made on the host, their synchronous upload, two transposing copies
+// and two indexed stores (a two-layer model's prefill of 1061 tokens and 8 decode steps, this and
+// q and k rotated in one launch: 8.8 -> 7.5 ms).
+__global__ __launch_bounds__(256) void append_tokens_kernel(int B, int L, int Hkv, SeqAddr kn, SeqAddr vn, KvAddr kc,
+                                                            KvAddr vc, int64_t start) {
+    const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int c = static_cast<int>(gid & 15);
+    const int64_t rt = gid >> 4;  // (b * L + t) * Hkv + h
+    const int64_t bt = rt / Hkv;
+    const int h = static_cast<int>(rt - bt * Hkv);
+    const int b = static_cast<int>(bt / L);
+    const int t = static_cast<int>(bt - (int64_t)b * L);
+    if (b >= B) return;
+    const int64_t pos = start + t;
+    const int64_t kb = pos >> 6;
+    const int off = static_cast<int>(pos & 63);
+    const int64_t row = (int64_t)b * Hkv + h;
+    const int64_t kphys = kc.page_table ? clamp_page(kc.page_table[row * kc.pts + kb], kc.max_page) : kb;
+    const int64_t vphys = vc.page_table ? clamp_page(vc.page_table[row * vc.pts + kb], vc.max_page) : kb;
+    const u32x4_v k = *reinterpret_cast<const u32x4_v*>(kn.data + b * kn.sb + (int64_t)t * kn.st + h * kn.sh + 8 * c);
+    const u32x4_v v = *reinterpret_cast<const u32x4_v*>(vn.data + b * vn.sb + (int64_t)t * vn.st + h * vn.sh + 8 * c);
+    *reinterpret_cast<u32x4_v*>(kc.data + b * kc.sb + h * kc.sh + kphys * kc.sblk + off * kc.stok + 8 * c) = k;
+    *reinterpret_cast<u32x4_v*>(vc.data + b * vc.sb + h * vc.sh + vphys * vc.sblk + off * vc.stok + 8 * c) = v;
 }
 
 }  // namespace
@@ -1440,6 +1486,18 @@ hipError_t launch_table_csr(const int32_t* table, int64_t table_stride, const in
 
 size_t union_lds_bytes(const Shape& s) { return sizeof(uint32_t) * (size_t)(s.G + 1) * s.words; }
 
+static hipError_t launch_union(const UnionParams& u, int last_n_block, hipStream_t stream) {
+    UnionParams p = u;
+    int tail = 0;
+    if (p.s.Qb > 1) {
+        tail = last_n_block < 0 ? 0 : last_n_block;
+        if (tail > p.s.Qb - 1) tail = p.s.Qb - 1;
+    }
+    p.pooled = p.s.Qb - tail;
+    hipLaunchKernelGGL(union_compact_kernel, dim3(p.s.B * p.s.Hkv), dim3(256), union_lds_bytes(p.s), stream, p);
+    return hipGetLastError();
+}
+
 hipError_t launch_union_compact(const Shape& s, const uint32_t* rowmask, int last_n_block,
                                 const uint8_t* keep_kv_in, const PastBlocks& pb, uint8_t* keep_block,
                                 uint8_t* keep_kv, int32_t* table, int64_t table_stride,
@@ -1449,20 +1507,44 @@ hipError_t launch_union_compact(const Shape& s, const uint32_t* rowmask, int las
     p.rowmask = rowmask;
     p.keep_kv_in = keep_kv_in;
     p.mode = dense ? 2 : (keep_kv_in ? 1 : 0);
-    int tail = 0;
-    if (s.Qb > 1) {
-        tail = last_n_block < 0 ? 0 : last_n_block;
-        if (tail > s.Qb - 1) tail = s.Qb - 1;
-    }
-    p.pooled = s.Qb - tail;
     p.pb = pb;
     p.keep_block = keep_block;
     p.keep_kv = keep_kv;
     p.table = table;
     p.table_stride = table_stride;
     p.counts = counts;
-    const size_t lds = union_lds_bytes(s);
-    hipLaunchKernelGGL(union_compact_kernel, dim3(s.B * s.Hkv), dim3(256), lds, stream, p);
+    p.pages = nullptr;
+    return launch_union(p, last_n_block, stream);
+}
+
+hipError_t launch_union_compact_pairs(const Shape& s, const uint32_t* rowmask, int last_n_block, const PastBlocks& pb,
+                                      int32_t* table, int64_t table_stride, int32_t* counts, int key_pages,
+                                      int32_t* pages, int64_t pages_stride, int page_cap, int32_t* page_counts,
+                                      hipStream_t stream) {
+    UnionParams p;
+    p.s = s;
+    p.rowmask = rowmask;
+    p.keep_kv_in = nullptr;
+    p.mode = 0;
+    p.pb = pb;
+    p.keep_block = nullptr;
+    p.keep_kv = nullptr;
+    p.table = table;
+    p.table_stride = table_stride;
+    p.counts = counts;
+    p.pages = pages;
+    p.pages_stride = pages_stride;
+    p.page_counts = page_counts;
+    p.key_pages = key_pages;
+    p.page_cap = page_cap;
+    return launch_union(p, last_n_block, stream);
+}
+
+hipError_t launch_append_tokens(int B, int L, int Hkv, const SeqAddr& k_new, const SeqAddr& v_new,
+                                const KvAddr& k_cache, const KvAddr& v_cache, int64_t start, hipStream_t stream) {
+    const int64_t threads = (int64_t)B * Hkv * L * (kD / 8);
+    hipLaunchKernelGGL(append_tokens_kernel, dim3(static_cast<unsigned>((threads + 255) / 256)), dim3(256), 0, stream, B,
+                       L, Hkv, k_new, v_new, k_cache, v_cache, start);
     return hipGetLastError();
 }
 

@@ -43,6 +43,12 @@ BLOCK = 64
 HEAD_DIM = 128
 
 
+def _kernel_rows(t: torch.Tensor) -> torch.Tensor:
+    """t itself when the append kernel can read it (16-byte rows at positive strides), else a copy."""
+    ok = t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all(s > 0 and s % 8 == 0 for s in t.stride()[:-1])
+    return t if ok else t.contiguous()
+
+
 class PagePool:
     """Grow-only pool of 64-token K and V pages with reference counts."""
 
@@ -285,13 +291,14 @@ class PagedKVCache:
         self._map(start // BLOCK, -(-end // BLOCK))
         if start % BLOCK:
             self._unshare(start // BLOCK)
-        pos = np.arange(start, end)
-        pages = self._pt[:, pos // BLOCK].astype(np.int64)  # [rows, L]
-        flat = torch.from_numpy(pages * BLOCK + (pos % BLOCK)[None, :]).to(self.device)
-        kf = self.pool.k.view(-1, HEAD_DIM)
-        vf = self.pool.v.view(-1, HEAD_DIM)
-        kf[flat.reshape(-1)] = k_new.transpose(1, 2).reshape(-1, HEAD_DIM)
-        vf[flat.reshape(-1)] = v_new.transpose(1, 2).reshape(-1, HEAD_DIM)
+        if self.device.type == "cpu":  # a cache in host memory (its kernels do not exist): plain indexing
+            pos = np.arange(start, end)
+            flat = torch.from_numpy(self._pt[:, pos // BLOCK].astype(np.int64) * BLOCK + (pos % BLOCK)[None, :])
+            for pool, new in ((self.pool.k, k_new), (self.pool.v, v_new)):
+                pool.view(-1, HEAD_DIM)[flat.reshape(-1)] = new.transpose(1, 2).reshape(-1, HEAD_DIM)
+        else:
+            K, V = self.layouts()
+            ops.append_tokens(_kernel_rows(k_new), _kernel_rows(v_new), K, V, start, self.cap)
         self.length = end
         return start
 

@@ -56,22 +56,6 @@ def check_score_block_size(block_size: int) -> None:
         raise ValueError(f"block_size={block_size}: FlashPrefill scoring runs 64- or 128-token blocks")
 
 
-def expand_pair_tables(table: torch.Tensor, counts: torch.Tensor, key_blocks: int, kv_cap: int
-                       ) -> Tuple[torch.Tensor, torch.Tensor]:
-    """Tables of 128-token blocks -> tables of 64-token pages: block k names pages 2k and 2k + 1,
-    in order; when key_blocks (the 64-token blocks of each row) is odd, the last 128-token block
-    (the current chunk's, closing every row) has page 2k only.  Entries past the counts are -1."""
-    rows = table.shape[0]
-    t = table.to(torch.int64)
-    pages = torch.stack([2 * t, 2 * t + 1], dim=-1).reshape(rows, -1)
-    cnt = 2 * counts.to(torch.int64) - (key_blocks % 2)
-    out = torch.full((rows, kv_cap), -1, dtype=torch.int32, device=table.device)
-    width = min(kv_cap, pages.shape[1])
-    keep = torch.arange(width, device=table.device)[None, :] < cnt[:, None]
-    out[:, :width] = torch.where(keep, pages[:, :width], torch.full_like(pages[:, :width], -1)).to(torch.int32)
-    return out, cnt.to(torch.int32)
-
-
 SCORE_MODES = ("pooled", "token")
 
 
@@ -130,8 +114,8 @@ def flashprefill_tables(qhat: torch.Tensor, khat: torch.Tensor, past_blocks: Seq
         rowmask = token_mass_rowmask(query_states, k128, P128, num_kv_heads, cap128, rule, 128)
     else:
         rowmask, _ = ops.score_select(q128, k128, scale, rule, P128, num_kv_heads, cap128)
-    t128, c128, _, _ = ops.union_compact(rowmask, P128, num_kv_heads, cap128, last_n_block=rule.last_n_block)
-    return expand_pair_tables(t128, c128, kb64, kv_cap)
+    return ops.union_compact(rowmask, P128, num_kv_heads, cap128, last_n_block=rule.last_n_block,
+                             pages=(kb64, kv_cap))[4:]
 
 
 def flashprefill_compactattn_prefill_full_kv(

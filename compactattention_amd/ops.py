@@ -226,6 +226,20 @@ def cache_fill(k_new: torch.Tensor, v_new: Optional[torch.Tensor], k_cache: Opti
                                    _ptr(rope_sin), rope_rows, _ptr(kgate), _stream()))
 
 
+def append_tokens(k_new: torch.Tensor, v_new: torch.Tensor, k_cache: KV, v_cache: KV, start: int, kv_cap: int) -> None:
+    """Write the tokens of k_new / v_new [B, L, Hkv, 128] at positions start .. start + L - 1 of
+    every request's rows (a decode append; no block summaries)."""
+    B, L, Hkv, _ = k_new.shape
+    kn, vn = seq_layout(k_new, "k_new"), seq_layout(v_new, "v_new")
+    if tuple(v_new.shape) != tuple(k_new.shape):
+        raise ValueError("v_new must have k_new's shape")
+    for name, kv in (("k", k_cache), ("v", v_cache)):
+        kv.check_blocks(name, B, Hkv, -(-(start + L) // BLOCK), tokens=start + L)
+    d = make_dims(B, L, Hkv, Hkv, kv_cap)
+    check(_hip.lib().ca_append_tokens(ctypes.byref(d), ctypes.byref(kn), ctypes.byref(vn), ctypes.byref(k_cache.layout),
+                                      ctypes.byref(v_cache.layout), int(start), _stream()))
+
+
 def pool_query(q: torch.Tensor, past_blocks: Sequence[int], kv_cap: int, gate_wq: Optional[torch.Tensor] = None,
                rope_cos: Optional[torch.Tensor] = None, rope_sin: Optional[torch.Tensor] = None,
                num_kv_heads: Optional[int] = None) -> torch.Tensor:
@@ -450,8 +464,14 @@ def select_scores(scores: torch.Tensor, rule: Rule, past_blocks: Sequence[int], 
 
 
 def union_compact(rowmask: torch.Tensor, past_blocks: Sequence[int], num_kv_heads: int, kv_cap: int,
-                  last_n_block: int = 0, want_keep_block: bool = False, want_keep_kv: bool = False):
-    """rowmask [B,Hq,Qb,words] -> (table [B*Hkv, kv_cap] i32, counts [B*Hkv] i32, keep_block, keep_kv)."""
+                  last_n_block: int = 0, want_keep_block: bool = False, want_keep_kv: bool = False,
+                  pages: Optional[Tuple[int, int]] = None):
+    """rowmask [B,Hq,Qb,words] -> (table [B*Hkv, kv_cap] i32, counts [B*Hkv] i32, keep_block, keep_kv).
+
+    ``pages`` = (key_pages, page_cap) with 128-token blocks (rowmask, past_blocks and kv_cap count
+    them): the tables in 64-token pages follow, (page table [B*Hkv, page_cap] i32, counts) --
+    block k names pages 2k and 2k + 1, the last block page 2k only when key_pages (the pages of
+    each row) is odd."""
     _need_cuda("rowmask", rowmask, torch.int32)
     if rowmask.dim() != 4 or rowmask.shape[3] != words_for(kv_cap) or not rowmask.is_contiguous():
         raise ValueError(f"rowmask must be contiguous [B, Hq, Qb, {words_for(kv_cap)}] int32")
@@ -460,6 +480,17 @@ def union_compact(rowmask: torch.Tensor, past_blocks: Sequence[int], num_kv_head
     dev = rowmask.device
     table = torch.empty((B * num_kv_heads, kv_cap), dtype=torch.int32, device=dev)
     counts = torch.empty((B * num_kv_heads,), dtype=torch.int32, device=dev)
+    if pages is not None:
+        if want_keep_block or want_keep_kv:
+            raise ValueError("the keep masks are not written beside page tables")
+        key_pages, page_cap = (int(x) for x in pages)
+        ptab = torch.empty((B * num_kv_heads, page_cap), dtype=torch.int32, device=dev)
+        pcnt = torch.empty((B * num_kv_heads,), dtype=torch.int32, device=dev)
+        check(_hip.lib().ca_union_compact_pairs(ctypes.byref(d), rowmask.data_ptr(), int(last_n_block),
+                                                past_array(past_blocks, d.batch), table.data_ptr(), table.stride(0),
+                                                counts.data_ptr(), key_pages, ptab.data_ptr(), ptab.stride(0), page_cap,
+                                                pcnt.data_ptr(), _stream()))
+        return table, counts, None, None, ptab, pcnt
     keep_block = torch.empty((B, Hq, kv_cap), dtype=torch.uint8, device=dev) if want_keep_block else None
     keep_kv = torch.empty((B, num_kv_heads, kv_cap), dtype=torch.uint8, device=dev) if want_keep_kv else None
     check(_hip.lib().ca_union_compact(ctypes.byref(d), rowmask.data_ptr(), int(last_n_block),
@@ -620,21 +651,41 @@ def attn_decode(q: torch.Tensor, k: KV, v: KV, kv_len: Sequence[int], scale: flo
 
 
 # ----------------------------------------------------------------------------- model plumbing
+def _rope_tables(cos: torch.Tensor, sin: torch.Tensor, L: int) -> None:
+    for name, t in (("cos", cos), ("sin", sin)):
+        _need_cuda(name, t, torch.float32)
+        if t.shape != (L, HEAD_DIM) or not t.is_contiguous():
+            raise ValueError(f"{name} must be contiguous fp32 [{L}, {HEAD_DIM}]")
+
+
 def rope(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """bf16(x * cos + rotate_half(x) * sin) for x [B, L, H, 128] bf16 and fp32 cos/sin [L, 128];
     bit-identical to apply_rotary_pos_emb evaluated in fp32."""
     B, L, H, _ = x.shape
     xl = seq_layout(x, "x")
-    for name, t in (("cos", cos), ("sin", sin)):
-        _need_cuda(name, t, torch.float32)
-        if t.shape != (L, HEAD_DIM) or not t.is_contiguous():
-            raise ValueError(f"{name} must be contiguous fp32 [{L}, {HEAD_DIM}]")
+    _rope_tables(cos, sin, L)
     if out is None:
         out = torch.empty((B, L, H, HEAD_DIM), dtype=torch.bfloat16, device=x.device)
     yl = seq_layout(out, "out")
     check(_hip.lib().ca_rope_apply(ctypes.byref(xl), ctypes.byref(yl), B, L, H, cos.data_ptr(), sin.data_ptr(),
                                    _stream()))
     return out
+
+
+def rope_qk(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
+    """(rope(q, cos, sin), rope(k, cos, sin)) in one launch."""
+    B, L, Hq, _ = q.shape
+    Hkv = k.shape[2]
+    ql, kl = seq_layout(q, "q"), seq_layout(k, "k")
+    if tuple(k.shape[:2]) != (B, L):
+        raise ValueError("q and k must cover the same [B, L] tokens")
+    _rope_tables(cos, sin, L)
+    qo = torch.empty((B, L, Hq, HEAD_DIM), dtype=torch.bfloat16, device=q.device)
+    ko = torch.empty((B, L, Hkv, HEAD_DIM), dtype=torch.bfloat16, device=k.device)
+    qol, kol = seq_layout(qo, "q_out"), seq_layout(ko, "k_out")
+    check(_hip.lib().ca_rope_qk(ctypes.byref(ql), ctypes.byref(qol), Hq, ctypes.byref(kl), ctypes.byref(kol), Hkv, B, L,
+                                cos.data_ptr(), sin.data_ptr(), _stream()))
+    return qo, ko
 
 
 def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float, residual: Optional[torch.Tensor] = None):

@@ -164,9 +164,10 @@ def project_qkv(attn: nn.Module, hidden_states: torch.Tensor) -> Tuple[torch.Ten
 
 def rope_qk(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor
             ) -> Tuple[torch.Tensor, torch.Tensor]:
-    """apply_rotary_pos_emb through the HIP rotary kernel (bit-identical results)."""
+    """apply_rotary_pos_emb through the HIP rotary kernel, q and k in one launch (bit-identical
+    results)."""
     cos, sin = cos.float().contiguous(), sin.float().contiguous()
-    return ops.rope(q, cos, sin), ops.rope(k, cos, sin)
+    return ops.rope_qk(q, k, cos, sin)
 
 
 def dense_decode_forward(attn: nn.Module, hidden_states: torch.Tensor, position_embeddings, cache: PagedKVCache):

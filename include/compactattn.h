@@ -164,6 +164,14 @@ int ca_cache_fill_pool_query(const ca_dims* dims, const ca_seq_layout* k_new, co
                              void* stream);
 
 /*
+ * Decode append: the q_len new tokens of every request (k_new / v_new, [B, q_len, Hkv, 128] bf16)
+ * at positions start .. start + q_len - 1 of the cache (uses dims->batch, q_len, num_kv_heads and
+ * kv_cap).  start need not be a multiple of 64; no block summaries are written.
+ */
+int ca_append_tokens(const ca_dims* dims, const ca_seq_layout* k_new, const ca_seq_layout* v_new,
+                     const ca_kv_layout* k_cache, const ca_kv_layout* v_cache, int64_t start, void* stream);
+
+/*
  * AttnGate block summaries for every gate type of the reference (compact_attn/prefill_sparse/
  * attn_gate.py:37-130,233-278: the Q{pools}_K{pools} classes, force_double, the
  * kv_group_aware_query form).  pools is a set of CA_POOL_* bits; the pooled vectors of a
@@ -284,6 +292,17 @@ int ca_select_scores(const ca_dims* dims, const void* scores, int32_t dtype, int
 int ca_union_compact(const ca_dims* dims, const uint32_t* rowmask, int32_t last_n_block,
                      const int32_t* past_blocks_host, uint8_t* keep_block, uint8_t* keep_kv,
                      int32_t* table, int64_t table_stride, int32_t* counts, void* stream);
+
+/*
+ * ca_union_compact over 128-token blocks (dims, past_blocks, rowmask and table count them), with the
+ * tables in 64-token page ids beside it: block k names pages 2k and 2k + 1 in order, and the last
+ * block, which closes every row, page 2k only when key_pages (the pages of every row) is odd.
+ * Rows of pages hold page_cap entries, -1 from page_counts[row] on.
+ */
+int ca_union_compact_pairs(const ca_dims* dims, const uint32_t* rowmask, int32_t last_n_block,
+                           const int32_t* past_blocks_host, int32_t* table, int64_t table_stride, int32_t* counts,
+                           int32_t key_pages, int32_t* pages, int64_t pages_stride, int32_t page_cap,
+                           int32_t* page_counts, void* stream);
 
 /*
  * Union + compaction from a caller-provided per-KV-group keep mask keep_kv
@@ -412,6 +431,11 @@ int64_t ca_attn_decode_workspace_size(const ca_dims* dims, const int32_t* kv_len
  */
 int ca_rope_apply(const ca_seq_layout* x, const ca_seq_layout* y, int32_t batch, int32_t len, int32_t heads,
                   const float* cos, const float* sin, void* stream);
+
+/* ca_rope_apply of q and k (the same tokens, their own head counts) in one launch. */
+int ca_rope_qk(const ca_seq_layout* q, const ca_seq_layout* q_out, int32_t q_heads, const ca_seq_layout* k,
+               const ca_seq_layout* k_out, int32_t k_heads, int32_t batch, int32_t len, const float* cos,
+               const float* sin, void* stream);
 int ca_rmsnorm(const uint16_t* x, int64_t x_stride, const uint16_t* residual, int64_t r_stride, uint16_t* sum_out,
                int64_t s_stride, const uint16_t* w, uint16_t* y, int64_t y_stride, int64_t rows, int32_t n, float eps,
                void* stream);
