@@ -344,7 +344,7 @@ __global__ __launch_bounds__(64 * NQ) void block_logits_kernel(Shape s, const fl
     for (int i = 0; i < CQ; ++i)
 #pragma unroll
         for (int j = 0; j < CK; ++j) acc[i][j] = f32x4_v{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll 8
+#pragma unroll
     for (int d = 0; d < kD; d += 4) {
         f32x4_v a[CQ], c[CK];
 #pragma unroll
