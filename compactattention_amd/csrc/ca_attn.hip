@@ -849,7 +849,10 @@ constexpr int kDecRows = 16;
 constexpr int kDecVBytes = 64 * 256;
 constexpr int kDecOStride = 132;  // floats per row of a wave's partial O in LDS (padded)
 
+// kStream: K and V are loaded with the non-temporal hint (when: launch_attn).
+template <bool kStream>
 __global__ __launch_bounds__(kDecWaves * 64) void attn_decode_kernel(AttnParams p) {
+    constexpr int kCache = kStream ? 2 : 0;  // cache policy of the loads: nt
     __shared__ __attribute__((aligned(16))) uint8_t smem[kDecWaves * kDecVBytes];
 
     const Shape& s = p.s;
@@ -951,11 +954,11 @@ __global__ __launch_bounds__(kDecWaves * 64) void attn_decode_kernel(AttnParams 
         for (int j = 0; j < 4; ++j)
 #pragma unroll
             for (int kt = 0; kt < 2; ++kt)
-                kf[set][kt][j] = __builtin_amdgcn_raw_buffer_load_b128(rk, kh + k_off[kt] + 64 * j, 0, 0);
+                kf[set][kt][j] = __builtin_amdgcn_raw_buffer_load_b128(rk, kh + k_off[kt] + 64 * j, 0, kCache);
 #pragma unroll
         for (int i = 0; i < 8; ++i)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, to_lds(vhalf[set] + i * 1024), 16,
-                                                     vh + v_goff[i & 1] + 4 * i * vstok_b, 0, 0, 0);
+                                                     vh + v_goff[i & 1] + 4 * i * vstok_b, 0, 0, kCache);
     };
 
     const float sl2 = p.scale_log2;
@@ -1338,11 +1341,20 @@ hipError_t launch_attn(const AttnArgs& a, hipStream_t stream) {
                     a.v.sblk == 64 * a.v.stok && (int64_t)max_tokens * stok * 2 + 64 * stok * 2 < (int64_t{1} << 31);
     }
     auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(p.per_xcd * 8), dim3(kNW * 64), 0, stream, p); };
+    // A decode launch reads its K and V once.  From the size of the last-level cache (256 MB) on,
+    // little of them is left there for a next launch, and loads that do not allocate in it are
+    // faster: 8 heads x 131072 tokens (537 MB) 100.4 us, 89.6 us non-temporal; ragged (508 MB)
+    // 102.2, 91.5; 65536 tokens (268 MB), three caches in turn 55.8, 51.8, one cache again and
+    // again 49.3, 50.5.  Below it a cache read again soon is found there: 49152 tokens in turn
+    // 45.3, 42.2, again and again 38.8, 41.2; four 4096-token requests (67 MB) 18.9, 19.4.
+    constexpr int64_t kLastLevelCache = int64_t{256} << 20;
+    int64_t kv_bytes = 0;
+    for (int b = 0; a.kv_len != nullptr && b < a.s.B; ++b) kv_bytes += (int64_t)a.kv_len[b] * a.s.Hkv * (2 * kD * 2);
     static_assert(kNW == kDecWaves, "one workgroup size for the attention kernels");
     if (a.table)
         row_res ? launch(attn_fwd_kernel<kNW, true, true>) : launch(attn_fwd_kernel<kNW, true, false>);
     else if (attn_uses_decode_kernel(a.s, true))
-        launch(attn_decode_kernel);
+        kv_bytes >= kLastLevelCache ? launch(attn_decode_kernel<true>) : launch(attn_decode_kernel<false>);
     else
         row_res ? launch(attn_fwd_kernel<kNW, false, true>) : launch(attn_fwd_kernel<kNW, false, false>);
     hipError_t e = hipGetLastError();

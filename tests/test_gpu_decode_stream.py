@@ -1,0 +1,50 @@
+"""Dense decode on both sides of the cache size above which K and V are loaded without staying in
+the last-level cache (2^28 bytes of K and V: 65536 tokens of 8 heads)."""
+from __future__ import annotations
+
+import math
+
+import pytest
+import torch
+
+from compactattention_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("layout", ["heads_first", "seq_first", "paged"])
+@pytest.mark.parametrize("lens", [[64001, 1534], [64001, 1535], [40000, 25600, 77]])
+def test_decode_around_the_cache_size(gpu, lens, layout):
+    print(f"case: decode lens={lens} layout={layout}", flush=True)
+    g = torch.Generator(device=gpu).manual_seed(sum(lens))
+    B, Hq, Hkv, cap = len(lens), 32, 8, (max(lens) + 63) // 64
+    q = torch.randn((B, 1, Hq, 128), generator=g, device=gpu).to(torch.bfloat16)
+    k, v = (torch.randn((B, Hkv, cap * 64, 128), generator=g, device=gpu).to(torch.bfloat16) for _ in range(2))
+    for b, n in enumerate(lens):  # rows past the request's last token are never used
+        k[b, :, n:] = float("nan")
+        v[b, :, n:] = float("nan")
+    if layout == "heads_first":
+        K, V = ops.KV.heads_first(k), ops.KV.heads_first(v)
+    elif layout == "seq_first":
+        K, V = (ops.KV.seq_first(t.transpose(1, 2).contiguous()) for t in (k, v))
+    else:
+        perm = torch.randperm(B * Hkv * cap, generator=g, device=gpu)
+        pools = []
+        for t in (k, v):
+            pool = torch.empty((B * Hkv * cap, 64, 128), dtype=torch.bfloat16, device=gpu)
+            pool[perm] = t.view(-1, 64, 128)
+            pools.append(pool)
+        pages = perm.to(torch.int32).view(B * Hkv, cap)
+        K, V = ops.KV.paged(pools[0], pages), ops.KV.paged(pools[1], pages)
+    scale = 1.0 / math.sqrt(128)
+    out, lse = ops.attn_decode(q, K, V, lens, scale, cap, Hkv, with_lse=True)
+    for b, n in enumerate(lens):
+        qf = q[b, 0].float().view(Hkv, Hq // Hkv, 128)
+        for h in range(Hkv):
+            s = (qf[h] @ k[b, h, :n].float().T.contiguous()) * scale
+            ref = torch.softmax(s, -1) @ v[b, h, :n].float()
+            err = (out[b, 0].float().view(Hkv, -1, 128)[h] - ref).abs()
+            # the attention tolerances: weights are rounded to bf16, an output is a mean under them
+            assert err.max() <= 2e-2 and err.mean() <= 2e-3, (b, h, err.max(), err.mean())
+            lerr = (lse[b].float().view(Hkv, -1)[h] - torch.logsumexp(s, -1)).abs().max()
+            assert lerr <= 4e-3, (b, h, lerr)
