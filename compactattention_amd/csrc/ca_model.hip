@@ -96,6 +96,10 @@ struct RmsParams {
     float eps;
 };
 
+// Bound by memory.  Nothing here is read twice from memory, so loads and stores are non-temporal:
+// the output stays out of the way of the product that reads it next.  512 rows of 4096 in a
+// norm -> gate/up product -> SwiGLU -> down product chain: 206 us, 203 us non-temporal (1024 rows
+// and more: no difference); 128 rows: 135.8, 134.8.
 constexpr int kRmsKeep = 4;  // chunks per thread held in registers: rows up to 8192 elements
 
 __global__ __launch_bounds__(256) void rmsnorm_kernel(RmsParams p) {
@@ -107,12 +111,12 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(RmsParams p) {
     const uint16_t* src = add ? p.s + row * p.s_stride : xr;
     // pass 1 over the thread's chunk i = 8 (t + 256 k): the (summed) row value, its square
     auto load = [&](int i, float& ss) {
-        u16x8_t v = *reinterpret_cast<const u16x8_t*>(xr + i);
+        u16x8_t v = __builtin_nontemporal_load(reinterpret_cast<const u16x8_t*>(xr + i));
         if (add) {
-            const u16x8_t rv = *reinterpret_cast<const u16x8_t*>(p.r + row * p.r_stride + i);
+            const u16x8_t rv = __builtin_nontemporal_load(reinterpret_cast<const u16x8_t*>(p.r + row * p.r_stride + i));
 #pragma unroll
             for (int j = 0; j < 8; ++j) v[j] = f32_to_bf16(bf16_to_f32(v[j]) + bf16_to_f32(rv[j]));
-            *reinterpret_cast<u16x8_t*>(p.s + row * p.s_stride + i) = v;
+            __builtin_nontemporal_store(v, reinterpret_cast<u16x8_t*>(p.s + row * p.s_stride + i));
         }
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
@@ -143,7 +147,7 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(RmsParams p) {
             const float yn = bf16_to_f32(f32_to_bf16(bf16_to_f32(v[j]) * rstd));
             o[j] = f32_to_bf16(bf16_to_f32(wv[j]) * yn);
         }
-        *reinterpret_cast<u16x8_t*>(yr + i) = o;
+        __builtin_nontemporal_store(o, reinterpret_cast<u16x8_t*>(yr + i));
     };
 #pragma unroll
     for (int k = 0; k < kRmsKeep; ++k) {
