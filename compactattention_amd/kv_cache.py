@@ -46,7 +46,7 @@ HEAD_DIM = 128
 def _kernel_rows(t: torch.Tensor) -> torch.Tensor:
     """t itself when the append kernel can read it (16-byte rows at positive strides), else a copy."""
     ok = t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all(s > 0 and s % 8 == 0 for s in t.stride()[:-1])
-    return t if ok else t.contiguous()
+    return t if ok else t.clone(memory_format=torch.contiguous_format)  # contiguous() keeps a misaligned start
 
 
 class PagePool:

@@ -23,10 +23,10 @@ def test_rope_qk_equals_two_calls(gpu, L, Hq, Hkv):
     assert torch.equal(qo, ops.rope(q, cos, sin)) and torch.equal(ko, ops.rope(k, cos, sin))
 
 
-@pytest.mark.parametrize("strided", ["dense", "heads_of_a_wider_row", "odd_strides"])
+@pytest.mark.parametrize("strided", ["dense", "heads_of_a_wider_row", "odd_strides", "misaligned"])
 def test_append_tokens_matches_indexing(gpu, strided):
     """Tokens on both sides of block edges, one and many at a time, next to a CPU cache's indexing;
-    rows the kernel cannot read in place (odd strides) go through a copy."""
+    rows the kernel cannot read in place (odd strides, a start that is not 16-byte aligned) go through a copy."""
     print(f"case: append_tokens {strided}", flush=True)
     g = torch.Generator().manual_seed(5)
     dev, host = PagedKVCache(2, 3, 64, gpu), PagedKVCache(2, 3, 64, "cpu")
@@ -37,6 +37,9 @@ def test_append_tokens_matches_indexing(gpu, strided):
             k, v = k.contiguous(), v.contiguous()
         xg = x.to(gpu)
         kg, vg = (k.to(gpu), v.to(gpu)) if strided == "dense" else (xg[..., :128], xg[..., 128:256])
+        if strided == "misaligned":  # contiguous tensors that start 2 bytes into an allocation
+            kg, vg = (torch.cat((t.new_zeros(1), t.reshape(-1)))[1:].view(t.shape) for t in (kg, vg))
+            assert kg.is_contiguous() and kg.data_ptr() % 16 != 0
         assert dev.append_tokens(kg, vg) == host.append_tokens(k, v)
     assert torch.equal(dev.k_hf().cpu(), host.k_hf()) and torch.equal(dev.v_hf().cpu(), host.v_hf())
 
