@@ -96,13 +96,23 @@ struct RmsParams {
     float eps;
 };
 
-// Bound by memory.  Nothing here is read twice from memory, so loads and stores are non-temporal:
-// the output stays out of the way of the product that reads it next.  512 rows of 4096 in a
-// norm -> gate/up product -> SwiGLU -> down product chain: 206 us, 203 us non-temporal (1024 rows
-// and more: no difference); 128 rows: 135.8, 134.8.
 constexpr int kRmsKeep = 4;  // chunks per thread held in registers: rows up to 8192 elements
 
+// Bound by memory.  kStream: rows held in registers are loaded and stored non-temporally, so they
+// stay out of the way of the product that reads the output next (when: launch_rmsnorm).
+template <bool kStream>
 __global__ __launch_bounds__(256) void rmsnorm_kernel(RmsParams p) {
+    auto get = [](const uint16_t* a) {
+        const u16x8_t* v = reinterpret_cast<const u16x8_t*>(a);
+        return kStream ? __builtin_nontemporal_load(v) : *v;
+    };
+    auto put = [](uint16_t* a, u16x8_t x) {
+        u16x8_t* v = reinterpret_cast<u16x8_t*>(a);
+        if (kStream)
+            __builtin_nontemporal_store(x, v);
+        else
+            *v = x;
+    };
     __shared__ float part[4];
     const int64_t row = blockIdx.x;
     const uint16_t* xr = p.x + row * p.x_stride;
@@ -111,12 +121,12 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(RmsParams p) {
     const uint16_t* src = add ? p.s + row * p.s_stride : xr;
     // pass 1 over the thread's chunk i = 8 (t + 256 k): the (summed) row value, its square
     auto load = [&](int i, float& ss) {
-        u16x8_t v = __builtin_nontemporal_load(reinterpret_cast<const u16x8_t*>(xr + i));
+        u16x8_t v = get(xr + i);
         if (add) {
-            const u16x8_t rv = __builtin_nontemporal_load(reinterpret_cast<const u16x8_t*>(p.r + row * p.r_stride + i));
+            const u16x8_t rv = get(p.r + row * p.r_stride + i);
 #pragma unroll
             for (int j = 0; j < 8; ++j) v[j] = f32_to_bf16(bf16_to_f32(v[j]) + bf16_to_f32(rv[j]));
-            __builtin_nontemporal_store(v, reinterpret_cast<u16x8_t*>(p.s + row * p.s_stride + i));
+            put(p.s + row * p.s_stride + i, v);
         }
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
@@ -147,7 +157,7 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(RmsParams p) {
             const float yn = bf16_to_f32(f32_to_bf16(bf16_to_f32(v[j]) * rstd));
             o[j] = f32_to_bf16(bf16_to_f32(wv[j]) * yn);
         }
-        __builtin_nontemporal_store(o, reinterpret_cast<u16x8_t*>(yr + i));
+        put(yr + i, o);
     };
 #pragma unroll
     for (int k = 0; k < kRmsKeep; ++k) {
@@ -225,7 +235,16 @@ hipError_t launch_rmsnorm(const uint16_t* x, int64_t x_stride, const uint16_t* r
     p.y_stride = y_stride;
     p.n = n;
     p.eps = eps;
-    hipLaunchKernelGGL(rmsnorm_kernel, dim3(static_cast<unsigned>(rows)), dim3(256), 0, stream, p);
+    // Non-temporal up to 16 MB per tensor (half of the eight 4 MB L2s) and while a row fits the
+    // registers, with the residual: 2048 rows of 4096 14.9 -> 13.1 us, 512 of 4096 6.1 -> 5.5,
+    // 2048 of 2048 8.4 -> 7.9; 512 rows of 4096 in a norm -> product -> SwiGLU -> product chain
+    // 206 -> 203 us.  Beyond, caches that keep the rows are faster: 8192 rows of 4096 43.1 us, 47.0
+    // non-temporal, 2048 of 8192 25.9 and 26.7; longer rows are read again: 512 of 16384 18.3 and 21.8.
+    const bool stream_rows = n <= 2048 * kRmsKeep && rows * n <= int64_t{8} << 20;
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(rows)), dim3(256), 0, stream, p);
+    };
+    stream_rows ? launch(rmsnorm_kernel<true>) : launch(rmsnorm_kernel<false>);
     return hipGetLastError();
 }
 

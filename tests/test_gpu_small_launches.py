@@ -66,3 +66,18 @@ def test_page_tables_beside_block_tables(gpu, kb64, slack):
         assert int(pcounts[r]) == len(want)
     with pytest.raises(Exception, match="key_pages"):
         ops.union_compact(rowmask.to(gpu), P, Hkv, cap, pages=(kb64 + 2, kb64 + 2))
+
+
+@pytest.mark.parametrize("n", [2048, 8192, 8200])
+@pytest.mark.parametrize("residual", [False, True])
+def test_rmsnorm_same_rows_in_launches_of_any_size(gpu, n, residual):
+    """Launches above the size that is streamed past the caches give the rows of launches below it."""
+    print(f"case: rmsnorm n={n} residual={residual}", flush=True)
+    rows = (8 << 20) // n + 1
+    g = torch.Generator(device=gpu).manual_seed(n)
+    x, r = (torch.randn((rows, n), generator=g, device=gpu).to(torch.bfloat16) for _ in range(2))
+    w = torch.randn((n,), generator=g, device=gpu).to(torch.bfloat16)
+    norm = lambda a, b: torch.stack(ops.rmsnorm(a, w, 1e-5, residual=b)) if residual else ops.rmsnorm(a, w, 1e-5)  # noqa: E731
+    whole = norm(x, r)
+    for part in (slice(0, rows - 1), slice(rows - 1, rows), slice(3, 70)):
+        assert torch.equal(whole[..., part, :], norm(x[part], r[part]))
