@@ -1341,20 +1341,20 @@ hipError_t launch_attn(const AttnArgs& a, hipStream_t stream) {
                     a.v.sblk == 64 * a.v.stok && (int64_t)max_tokens * stok * 2 + 64 * stok * 2 < (int64_t{1} << 31);
     }
     auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(p.per_xcd * 8), dim3(kNW * 64), 0, stream, p); };
-    // A decode launch reads its K and V once.  From the size of the last-level cache (256 MB) on,
-    // little of them is left there for a next launch, and loads that do not allocate in it are
-    // faster: 8 heads x 131072 tokens (537 MB) 100.4 us, 89.6 us non-temporal; ragged (508 MB)
-    // 102.2, 91.5; 65536 tokens (268 MB), three caches in turn 55.8, 51.8, one cache again and
-    // again 49.3, 50.5.  Below it a cache read again soon is found there: 49152 tokens in turn
-    // 45.3, 42.2, again and again 38.8, 41.2; four 4096-token requests (67 MB) 18.9, 19.4.
-    constexpr int64_t kLastLevelCache = int64_t{256} << 20;
+    // A decode launch reads its K and V once.  When they are a good deal more than the last-level
+    // cache (256 MB) holds, nothing useful of them is left there for a next launch, and loads that
+    // do not allocate in it are faster: 8 heads x 131072 tokens (537 MB) 100.4 us, 89.6 us
+    // non-temporal; 81920 tokens (336 MB) 64.0, 60.4.  Nearer to its size a cache read again at
+    // once is partly found there: 73728 tokens 54.7, 55.2; 49152 38.8, 41.2; four 4096-token
+    // requests (67 MB) 18.9, 19.4 (several caches in turn: 73728 tokens 61.0, 55.8; 49152 45.3, 42.2).
+    constexpr int64_t kStreamBytes = int64_t{320} << 20;
     int64_t kv_bytes = 0;
     for (int b = 0; a.kv_len != nullptr && b < a.s.B; ++b) kv_bytes += (int64_t)a.kv_len[b] * a.s.Hkv * (2 * kD * 2);
     static_assert(kNW == kDecWaves, "one workgroup size for the attention kernels");
     if (a.table)
         row_res ? launch(attn_fwd_kernel<kNW, true, true>) : launch(attn_fwd_kernel<kNW, true, false>);
     else if (attn_uses_decode_kernel(a.s, true))
-        kv_bytes >= kLastLevelCache ? launch(attn_decode_kernel<true>) : launch(attn_decode_kernel<false>);
+        kv_bytes >= kStreamBytes ? launch(attn_decode_kernel<true>) : launch(attn_decode_kernel<false>);
     else
         row_res ? launch(attn_fwd_kernel<kNW, false, true>) : launch(attn_fwd_kernel<kNW, false, false>);
     hipError_t e = hipGetLastError();

@@ -1,5 +1,5 @@
-"""Dense decode on both sides of the cache size above which K and V are loaded without staying in
-the last-level cache (2^28 bytes of K and V: 65536 tokens of 8 heads)."""
+"""Dense decode on both sides of the size from which K and V are loaded without staying in the
+last-level cache (320 MB of K and V: 81920 tokens of 8 heads)."""
 from __future__ import annotations
 
 import math
@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("layout", ["heads_first", "seq_first", "paged"])
-@pytest.mark.parametrize("lens", [[64001, 1534], [64001, 1535], [40000, 25600, 77]])
+@pytest.mark.parametrize("lens", [[80001, 1918], [80001, 1919], [45000, 40000, 77]])
 def test_decode_around_the_cache_size(gpu, lens, layout):
     print(f"case: decode lens={lens} layout={layout}", flush=True)
     g = torch.Generator(device=gpu).manual_seed(sum(lens))
