@@ -198,12 +198,19 @@ __device__ __forceinline__ u32x4_t buffer_words(const uint16_t* base, int bytes)
                    static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(bytes)), 0x00020000u};
 }
 // One LDS-DMA load: lane L's 16 bytes at byte offset off of the resource go to LDS byte dst + 16 L.
+// A vector-memory instruction may read an SGPR five wait states after a vector instruction wrote it
+// at the earliest (v_readfirstlane and v_readlane do), and the compiler inserts none for
+// instructions of inline asm: the block brings all five itself (s_mov and s_nop 3), whatever comes
+// before it.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void dma_lds(u32x4_t rsrc, int off, uint32_t dst) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds"
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 3\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds"
                  :
                  : "v"(off), "s"(rsrc), "s"(dst)
-                 : "memory");
+                 : "memory", "m0");
 }
+#pragma clang diagnostic pop
 template <int N>
 struct IntC {
     static constexpr int value = N;

@@ -71,3 +71,69 @@ def test_list_lengths_partial_block_and_splits(gpu, layout):
     _case(gpu, [3, 66], 37, 14, 2, layout, 1)
     _case(gpu, [130, 7], 150, 14, 2, layout, 3)
     _case(gpu, [259, 200], 64, 8, 2, layout, 2)
+
+
+@pytest.mark.parametrize("Lq", [37, 64, 150])
+@pytest.mark.parametrize("splits", [0, 1, 2, 3])
+def test_page_pool_equals_heads_first(gpu, Lq, splits):
+    """Requests whose last blocks are different ids, partial where Lq is not a multiple of 64, with NaN
+    in every row past their last token: a page pool gives the heads-first cache's output bit for bit."""
+    print(f"case: page pool Lq={Lq} splits={splits}", flush=True)
+    Hq, Hkv, P = 14, 2, [0, 3, 70, 131]
+    B, Qb = len(P), -(-Lq // 64)
+    cap = max(P) + Qb
+    g = torch.Generator().manual_seed(Lq + splits)
+    q = torch.randn((B, Lq, Hq, 128), generator=g).to(torch.bfloat16).to(gpu)
+    k, v = (torch.randn((B, Hkv, cap * 64, 128), generator=g).to(torch.bfloat16).to(gpu) for _ in range(2))
+    keep = (torch.rand((B, Hkv, cap), generator=g) < 0.6).to(torch.uint8)
+    for b, past in enumerate(P):
+        k[b, :, 64 * past + Lq:] = float("nan")
+        v[b, :, 64 * past + Lq:] = float("nan")
+        keep[b, :, past:] = 0
+    table, counts = ops.compact_keep_kv(keep.to(gpu), P, Lq, Hq, cap)
+    perm = torch.randperm(B * Hkv * cap, generator=g).to(gpu)
+    pools = []
+    for t in (k, v):
+        pool = torch.empty((B * Hkv * cap, 64, 128), dtype=torch.bfloat16, device=gpu)
+        pool[perm] = t.view(-1, 64, 128)
+        pools.append(pool)
+    pages = perm.to(torch.int32).view(B * Hkv, cap)
+    scale = 1.0 / math.sqrt(128)
+    want, want_lse = ops.attn_fwd(q, ops.KV.heads_first(k), ops.KV.heads_first(v), table, counts, P, scale, cap, Hkv,
+                                  with_lse=True, num_splits=splits)
+    out, lse = ops.attn_fwd(q, ops.KV.paged(pools[0], pages), ops.KV.paged(pools[1], pages), table, counts, P, scale,
+                            cap, Hkv, with_lse=True, num_splits=splits)
+    assert torch.equal(out, want) and torch.equal(lse, want_lse)
+    k, v = k.nan_to_num(), v.nan_to_num()  # the reference gathers whole blocks (masked for every row)
+    torch_reference_check(out, q, k, v, P, table, counts, scale, lse=lse)
+
+
+def test_dense_decode_of_many_rows_through_a_page_pool(gpu):
+    """Decode with more packed rows than its own kernel holds: the block loop over identity lists."""
+    print("case: dense decode, 40 packed rows, page pool", flush=True)
+    Hq, Hkv, L, lens = 16, 2, 5, [5, 63, 131, 4500]
+    cap = -(-max(lens) // 64)
+    g = torch.Generator().manual_seed(1)
+    q = torch.randn((len(lens), L, Hq, 128), generator=g).to(torch.bfloat16).to(gpu)
+    k, v = (torch.randn((len(lens), Hkv, cap * 64, 128), generator=g).to(torch.bfloat16).to(gpu) for _ in range(2))
+    for b, n in enumerate(lens):
+        k[b, :, n:] = float("nan")
+        v[b, :, n:] = float("nan")
+    perm = torch.randperm(len(lens) * Hkv * cap, generator=g).to(gpu)
+    pools = []
+    for t in (k, v):
+        pool = torch.empty((len(perm), 64, 128), dtype=torch.bfloat16, device=gpu)
+        pool[perm] = t.view(-1, 64, 128)
+        pools.append(pool)
+    pages = perm.to(torch.int32).view(len(lens) * Hkv, cap)
+    scale = 1.0 / math.sqrt(128)
+    args = (lens, scale, cap, Hkv)
+    want = ops.attn_decode(q, ops.KV.heads_first(k), ops.KV.heads_first(v), *args)
+    out = ops.attn_decode(q, ops.KV.paged(pools[0], pages), ops.KV.paged(pools[1], pages), *args)
+    assert torch.equal(out, want)
+    for b, n in enumerate(lens):
+        for h in range(Hq):
+            s = (q[b, :, h].float() @ k[b, h * Hkv // Hq, :n].float().T.contiguous()) * scale
+            s.masked_fill_(torch.arange(n, device=gpu)[None, :] > torch.arange(n - L, n, device=gpu)[:, None], float("-inf"))
+            err = (out[b, :, h].float() - torch.softmax(s, -1) @ v[b, h * Hkv // Hq, :n].float()).abs()
+            assert err.max() <= 2e-2 and err.mean() <= 2e-3, (b, h, err.max(), err.mean())
