@@ -72,7 +72,7 @@ struct AttnParams {
     SeqAddr out;
     float* lse;
     int ntiles;       // packed-row tiles per KV row
-    int sp0;          // splits of the first request (of every one in kPlaceRows and kPlaceSplits)
+    int sp0;          // kPlaceSplits: splits of every request
     int rows_total;   // Lq * G
     int total_items;  // B*Hkv*ntiles*splits
     int per_xcd;      // ceil(total_items / 8)
@@ -88,6 +88,7 @@ struct AttnParams {
     int32_t ioff[CA_MAX_BATCH + 1];  // first work item of each request (linear placement)
     int placement;                   // kPlace*: where a workgroup finds its unit
     int units;                       // kPlaceSplits: units in all
+    int unit_splits;                 // kPlaceRows, kPlaceTable: the splits of every unit, 0 when they differ
     int32_t xoff[9];                 // kPlaceTable
     uint32_t unit[kPlanRows];
 };
@@ -98,36 +99,45 @@ struct Item {
     int row, b, split, tile;
 };
 // Workgroup L runs on XCD L % 8 and is that XCD's (L / 8)-th; false when the XCD has no such
-// item.  Equal requests need no table (kPlaceRows, kPlaceSplits: arithmetic); a ragged launch's
-// units are read 64 at a time, one per lane, and found by a prefix sum over their items, so the
-// search costs one read's latency and not one per unit.
+// item.  Where all units hold the same number of splits the unit's place is computed: equal
+// requests need no table (kPlaceRows, kPlaceSplits), a ragged launch reads one entry.  The units
+// of a ragged launch differ only when a decode has more than kPlanRows splits in all; those are
+// read 64 at a time, one per lane, and found by a prefix sum over their items.
+// Every workgroup starts with this, so its latency shows in short launches (decode, from graph
+// replays: a scalar scan over the units, the prefix sum in all ragged launches, this): 5 requests
+// of 254-23110 tokens, 8 / 8 heads 33.6, 34.6, 33.9 us; 4 of 460-42073, 16 / 2 heads 26.1, 26.5,
+// 25.8; 7 of 136-8722, 16 / 2 heads 15.8, 14.7, 14.1.
 __device__ __forceinline__ bool find_item(const AttnParams& p, int ntiles, Item* it) {
     const int x = blockIdx.x & 7;
     int k = blockIdx.x >> 3;
     const int Hkv = p.s.Hkv;
-    int lo = 0, cnt;
-    if (p.placement == kPlaceRows) {
-        cnt = p.sp0;
-        const int u = k / (ntiles * cnt);
-        it->row = x + 8 * u;
-        if (it->row >= p.s.B * Hkv) return false;
-        k -= u * ntiles * cnt;
-    } else if (p.placement == kPlaceSplits) {
-        cnt = 1;
-        const int u = x + 8 * (k / ntiles);
-        if (u >= p.units) return false;
-        it->row = u / p.sp0;
-        lo = u - it->row * p.sp0;
-        k %= ntiles;
+    int lo = 0, cnt = p.unit_splits;
+    auto unit = [&](uint32_t word) {
+        it->row = word & (kPlanRows - 1);
+        it->b = (word >> kUnitReq) & (CA_MAX_BATCH - 1);
+        lo = (word >> kUnitLo) & 0xffu;
+        cnt = word >> kUnitCnt;
+    };
+    if (cnt > 0) {
+        const int per = ntiles * cnt;
+        int u = k;
+        if (per != 1) u = k / per;  // (an integer division is a chain of about 0.1 us)
+        k -= u * per;
+        if (p.placement == kPlaceRows) {
+            it->row = x + 8 * u;
+            if (it->row >= p.s.B * Hkv) return false;
+            it->b = it->row / Hkv;
+        } else {
+            if (p.xoff[x] + u >= p.xoff[x + 1]) return false;
+            unit(p.unit[p.xoff[x] + u]);
+        }
     } else if (p.placement == kPlaceTable) {
         const int lane = threadIdx.x & 63;
         const int end = p.xoff[x + 1];
-        int base = p.xoff[x];
-        uint32_t word = 0;
-        for (;; base += 64) {
+        for (int base = p.xoff[x];; base += 64) {
             if (base >= end) return false;
             const uint32_t w = base + lane < end ? p.unit[base + lane] : 0u;
-            int sum = ntiles * static_cast<int>(w >> 24);  // inclusive prefix of the units' items
+            int sum = ntiles * static_cast<int>(w >> kUnitCnt);  // inclusive prefix of the units' items
 #pragma unroll
             for (int o = 1; o < 64; o <<= 1) {
                 const int y = __shfl_up(sum, o, 64);
@@ -136,28 +146,35 @@ __device__ __forceinline__ bool find_item(const AttnParams& p, int ntiles, Item*
             const int total = __builtin_amdgcn_readlane(sum, 63);
             if (k < total) {
                 const int u = __popcll(__ballot(sum <= k));
-                word = __builtin_amdgcn_readlane(w, u);
+                unit(__builtin_amdgcn_readlane(w, u));
                 if (u > 0) k -= __builtin_amdgcn_readlane(sum, u - 1);
                 break;
             }
             k -= total;
         }
-        it->row = word & 0xffffu;
-        lo = (word >> 16) & 0xffu;
-        cnt = word >> 24;
     } else {
-        const int W = x * p.per_xcd + k;
-        if (W >= p.total_items) return false;
-        int b = 0;
-        while (b + 1 < p.s.B && p.ioff[b + 1] <= W) ++b;
-        cnt = p.sp[b];
-        const int local = W - p.ioff[b];
-        const int u = local / (ntiles * cnt);
-        it->row = b * Hkv + u;
-        k = local - u * ntiles * cnt;
+        if (p.placement == kPlaceSplits) {
+            cnt = 1;
+            const int u = x + 8 * (k / ntiles);
+            if (u >= p.units) return false;
+            it->row = u / p.sp0;
+            lo = u - it->row * p.sp0;
+            k %= ntiles;
+        } else {
+            const int W = x * p.per_xcd + k;
+            if (W >= p.total_items) return false;
+            int b = 0;
+            while (b + 1 < p.s.B && p.ioff[b + 1] <= W) ++b;
+            cnt = p.sp[b];
+            const int local = W - p.ioff[b];
+            const int u = local / (ntiles * cnt);
+            it->row = b * Hkv + u;
+            k = local - u * ntiles * cnt;
+        }
+        it->b = it->row / Hkv;
     }
-    it->b = it->row / Hkv;
-    it->tile = k / cnt;
+    it->tile = k;
+    if (cnt != 1) it->tile = k / cnt;
     it->split = lo + k - it->tile * cnt;
     return true;
 }
@@ -282,7 +299,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
         const int per = (p.xoff[x + 1] - i0) * p.ntiles;  // items of one split on this XCD
         if (k >= per) return;  // the unsplit row's items are those of split 0
         const int i = k / p.ntiles;
-        it.row = p.unit[i0 + i] & 0xffffu;
+        it.row = p.unit[i0 + i] & (kPlanRows - 1);
         it.b = it.row / s.Hkv;
         it.split = 0;
         it.tile = k - i * p.ntiles;
@@ -1179,6 +1196,7 @@ void attn_plan(const Shape& s, const int32_t* nkb, int forced, bool dense, Split
     plan->sp0 = plan->s[0];
     plan->placement = kPlaceLinear;
     plan->units = 0;
+    plan->unit_splits = 0;
     plan->per_xcd = (plan->off[s.B] + 7) / 8;
     if (rows > kPlanRows) return;
     // Placement units on the 8 XCDs.  A unit is a KV row and a range of its splits; the row
@@ -1201,6 +1219,7 @@ void attn_plan(const Shape& s, const int32_t* nkb, int forced, bool dense, Split
     if (same_len && (rows % 8 == 0 || split_units)) {
         plan->placement = split_units ? kPlaceSplits : kPlaceRows;
         plan->units = split_units ? nunits : rows;
+        plan->unit_splits = split_units ? 0 : plan->sp0;
         plan->per_xcd = (plan->units + 7) / 8 * ntiles * (split_units ? 1 : plan->sp0);
         return;
     }
@@ -1221,6 +1240,9 @@ void attn_plan(const Shape& s, const int32_t* nkb, int forced, bool dense, Split
             ++units;
         }
     }
+    plan->unit_splits = unit_cnt[0];
+    for (int u = 1; u < units; ++u)
+        if (unit_cnt[u] != unit_cnt[0]) plan->unit_splits = 0;
     int xcd_of[kPlanRows];
     double load[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     int items[8] = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -1267,7 +1289,8 @@ void attn_plan(const Shape& s, const int32_t* nkb, int forced, bool dense, Split
     for (int x = 0; x < 8; ++x) {
         for (int i = 0; i < nunit[x]; ++i) {
             const int u = lists[x][i];
-            plan->unit[plan->xoff[x] + i] = static_cast<uint32_t>(unit_row[u] | unit_lo[u] << 16 | unit_cnt[u] << 24);
+            plan->unit[plan->xoff[x] + i] = static_cast<uint32_t>(
+                unit_row[u] | (unit_row[u] / s.Hkv) << kUnitReq | unit_lo[u] << kUnitLo | unit_cnt[u] << kUnitCnt);
         }
         plan->xoff[x + 1] = plan->xoff[x] + nunit[x];
         plan->per_xcd = max(plan->per_xcd, items[x]);
@@ -1329,6 +1352,7 @@ hipError_t launch_attn(const AttnArgs& a, hipStream_t stream) {
     p.placement = plan.placement;
     p.sp0 = plan.sp0;
     p.units = plan.units;
+    p.unit_splits = plan.unit_splits;
     if (plan.placement == kPlaceTable) {  // the kernels read the table in this case only
         for (int x = 0; x < 9; ++x) p.xoff[x] = plan.xoff[x];
         for (int i = 0; i < plan.xoff[8]; ++i) p.unit[i] = plan.unit[i];

@@ -118,18 +118,23 @@ constexpr int kMaxDecodeSplits = 64;
 //  - kPlaceSplits: requests of one length otherwise: split u % sp0 of row u / sp0 on XCD u % 8
 //    (a row's splits stream disjoint parts of its block list);
 //  - kPlaceTable: ragged launches: entries xoff[x] .. xoff[x+1] list XCD x's units in order, each
-//    a row and a range of its splits (unit: row | first split << 16 | splits << 24);
+//    a row and a range of its splits (unit: the row, from the kUnit* bits on its request, first
+//    split and split count);
 //  - kPlaceLinear: more than kPlanRows KV rows: items numbered request by request (off[b]) and
 //    dealt to XCDs in contiguous ranges.
 constexpr int kPlanRows = 512;
+constexpr int kUnitReq = 9, kUnitLo = 15, kUnitCnt = 23;
+static_assert(kPlanRows <= 1 << kUnitReq && CA_MAX_BATCH <= 1 << (kUnitLo - kUnitReq), "the fields of a unit");
+static_assert(kMaxDecodeSplits <= 255 && kMaxPrefillSplits <= 255, "the fields of a unit");
 enum { kPlaceLinear = 0, kPlaceRows = 1, kPlaceSplits = 2, kPlaceTable = 3 };
 struct SplitPlan {
     int32_t s[CA_MAX_BATCH];
     int32_t off[CA_MAX_BATCH + 1];
     int max;
     int placement;
-    int sp0;          // splits of the first request
+    int sp0;          // kPlaceSplits: splits of every request
     int units;        // kPlaceRows, kPlaceSplits
+    int unit_splits;  // kPlaceRows, kPlaceTable: the splits of every unit, 0 when they differ
     int per_xcd;      // work items per XCD (grid = 8 * per_xcd)
     int may_unsplit;  // the kernel drops the splits when the rows' selected counts are even
     uint32_t unit[kPlanRows];

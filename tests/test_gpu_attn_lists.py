@@ -137,3 +137,29 @@ def test_dense_decode_of_many_rows_through_a_page_pool(gpu):
             s.masked_fill_(torch.arange(n, device=gpu)[None, :] > torch.arange(n - L, n, device=gpu)[:, None], float("-inf"))
             err = (out[b, :, h].float() - torch.softmax(s, -1) @ v[b, h * Hkv // Hq, :n].float()).abs()
             assert err.max() <= 2e-2 and err.mean() <= 2e-3, (b, h, err.max(), err.mean())
+
+
+@pytest.mark.parametrize("lens,splits", [
+    ([4342, 42073, 460, 1201], 0),            # placement units of one split each
+    ([65, 2048, 300] + [200] * 54 + [2048, 2001, 130], 0),  # over 512 splits: whole rows, of 1 and of 3 splits
+    ([65, 2048, 300] + [200] * 54 + [2048, 2001, 130], 2),  # whole rows of two splits
+])
+def test_ragged_decode_placement(gpu, lens, splits):
+    """Every way a workgroup of a ragged launch finds its request, KV row and split."""
+    print(f"case: ragged decode B={len(lens)} splits={splits}", flush=True)
+    B, Hq, Hkv, cap = len(lens), 16, 8, -(-max(lens) // 64)
+    g = torch.Generator(device=gpu).manual_seed(B + splits)
+    q = torch.randn((B, 1, Hq, 128), generator=g, device=gpu).to(torch.bfloat16)
+    k, v = (torch.randn((B, Hkv, cap * 64, 128), generator=g, device=gpu).to(torch.bfloat16) for _ in range(2))
+    for b, n in enumerate(lens):
+        k[b, :, n:] = float("nan")
+        v[b, :, n:] = float("nan")
+    scale = 1.0 / math.sqrt(128)
+    out = ops.attn_decode(q, ops.KV.heads_first(k), ops.KV.heads_first(v), lens, scale, cap, Hkv, num_splits=splits)
+    for b, n in enumerate(lens):
+        for h in range(Hkv):
+            rows = q[b, 0, 2 * h:2 * h + 2].float()
+            s = (rows @ k[b, h, :n].float().T.contiguous()) * scale
+            err = (out[b, 0, 2 * h:2 * h + 2].float() - torch.softmax(s, -1) @ v[b, h, :n].float()).abs()
+            # the attention tolerances: weights are rounded to bf16, an output is a mean under them
+            assert err.max() <= 2e-2 and err.mean() <= 2e-3, (b, h, err.max(), err.mean())
