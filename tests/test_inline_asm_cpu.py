@@ -44,20 +44,43 @@ def functions(tmp_path_factory):
     return found
 
 
-def test_asm_loads_bring_their_wait_states(functions):
-    loads = 0
+def _sgprs(operand):
+    m = re.fullmatch(r"s\[(\d+):(\d+)\]|s(\d+)", operand)
+    return set() if m is None else {int(m[3])} if m[3] else set(range(int(m[1]), int(m[2]) + 1))
+
+
+def _vector_writes(op, args):
+    """SGPRs that a vector instruction may write (the first operand, or the second of those with a carry)."""
+    operands = [a.split()[0] for a in args.split(",")] if op.startswith("v_") else []
+    return set().union(*(_sgprs(a) for a in operands[:1 if re.match("v_read", op) else 2]))
+
+
+def test_asm_loads_have_their_wait_states(functions):
+    """Five wait states lie between a vector write of a load's SGPRs and the load: in its own asm block,
+    or the kernel waits them once ("s_nop 4") and no vector instruction writes those SGPRs from there on."""
+    whole, fixed = 0, 0
     for name, lines in functions.items():
+        loads, settled = [], None
         states = last = 0
-        for block, op, args in lines:
+        for i, (block, op, args) in enumerate(lines):
             if block != last:
                 states, last = 0, block  # what came before the block may have written its operands
             if not block:
                 continue
+            if (op, args) == ("s_nop", str(SGPR_READ_STATES - 1)):
+                settled = i
             if op.startswith(("buffer_", "global_", "scratch_", "flat_")):
-                loads += 1
-                assert states >= SGPR_READ_STATES, (name, op, args, states)
+                loads.append((i, states, set().union(*(_sgprs(a.split()[0]) for a in args.split(",")))))
             states += _states(op, args)
-    assert loads > 0
+        for i, states, read in loads:
+            if states >= SGPR_READ_STATES:
+                whole += 1
+                continue
+            fixed += 1
+            assert settled is not None and settled < i, (name, i, states)
+            for block, op, args in lines[settled + 1:loads[-1][0]]:
+                assert not read & _vector_writes(op, args), (name, op, args)
+    assert whole > 0 and fixed > 0
 
 
 def test_asm_blocks_have_m0_to_themselves(functions):
