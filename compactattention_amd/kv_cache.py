@@ -286,6 +286,9 @@ class PagedKVCache:
             raise ValueError("k_new does not match the cache's batch / KV heads")
         if L == 0:
             return self.length
+        device = self.pool.k.device
+        if k_new.device != device or v_new.device != device:
+            raise ValueError(f"k_new on {k_new.device} and v_new on {v_new.device} do not match the cache's {device}")
         start = self.length
         end = start + L
         self._map(start // BLOCK, -(-end // BLOCK))
@@ -298,7 +301,8 @@ class PagedKVCache:
                 pool.view(-1, HEAD_DIM)[flat.reshape(-1)] = new.transpose(1, 2).reshape(-1, HEAD_DIM)
         else:
             K, V = self.layouts()
-            ops.append_tokens(_kernel_rows(k_new), _kernel_rows(v_new), K, V, start, self.cap)
+            with torch.cuda.device(device):  # the cache's own, whichever is current
+                ops.append_tokens(_kernel_rows(k_new), _kernel_rows(v_new), K, V, start, self.cap)
         self.length = end
         return start
 

@@ -109,6 +109,43 @@ def test_paged_cache_decode_append_rules():
         c.append(k[:, :64], k[:, :64])
 
 
+def test_paged_cache_decode_append_runs_on_the_cache_s_device(monkeypatch):
+    """A decode append launches on the device that holds the cache, also while another one is current,
+    and refuses tokens that lie on another device."""
+    from contextlib import contextmanager
+    from types import SimpleNamespace
+
+    from compactattention_amd import kv_cache
+
+    second = torch.device("cuda", 1)
+
+    class OnSecond(torch.Tensor):
+        device = second
+
+    c = kv_cache.PagedKVCache(1, 2, 192, "cpu")
+    c.reserve(128)
+    c.device, c.pool.k = second, SimpleNamespace(device=second)
+    c.layouts = lambda: (None, None)
+    current, launched = [torch.device("cuda", 0)], []
+
+    @contextmanager
+    def device(d):
+        current.append(d)
+        yield
+        current.pop()
+
+    monkeypatch.setattr(kv_cache.torch.cuda, "device", device)
+    monkeypatch.setattr(kv_cache.ops, "append_tokens", lambda *args: launched.append(current[-1]))
+    k = torch.zeros((1, 3, 2, 128), dtype=torch.bfloat16)
+    there = k.as_subclass(OnSecond)
+    assert c.append_tokens(there, there) == 0 and c.length == 3
+    assert launched == [second] and len(current) == 1
+    for kn, vn in ((k, there), (there, k)):
+        with pytest.raises(ValueError, match="do not match the cache's cuda:1"):
+            c.append_tokens(kn, vn)
+    assert launched == [second] and c.length == 3
+
+
 def test_paged_cache_allocator_growth_fork_and_copy_on_write():
     """Host logic of the page pool and page table (CPU tensors; the kernels only read them):
     pages are handed out per (row, block) as the sequence grows, the pool and the page
