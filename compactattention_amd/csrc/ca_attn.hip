@@ -885,18 +885,14 @@ constexpr int kDecRows = 16;
 constexpr int kDecVBytes = 64 * 256;
 constexpr int kDecOStride = 132;  // floats per row of a wave's partial O in LDS (padded)
 
-// kStream: K and V are loaded with the non-temporal hint (when: launch_attn).
+// One work item.  kStream: K and V are loaded with the non-temporal hint.
 template <bool kStream>
-__global__ __launch_bounds__(kDecWaves * 64) void attn_decode_kernel(AttnParams p) {
+__device__ __forceinline__ void decode_item(const AttnParams& p, const Item& it, uint8_t* smem) {
     constexpr int kCache = kStream ? 2 : 0;  // cache policy of the loads: nt
-    __shared__ __attribute__((aligned(16))) uint8_t smem[kDecWaves * kDecVBytes];
-
     const Shape& s = p.s;
-    Item it;
-    if (!find_item(p, 1, &it)) return;
-    const int row = __builtin_amdgcn_readfirstlane(it.row);
-    const int b = __builtin_amdgcn_readfirstlane(it.b);
-    const int split = __builtin_amdgcn_readfirstlane(it.split);
+    const int row = it.row;
+    const int b = it.b;
+    const int split = it.split;
     const int hk = row - b * s.Hkv;
     const int nsplit = p.sp[b];
     const int G = s.G;
@@ -1123,6 +1119,36 @@ __global__ __launch_bounds__(kDecWaves * 64) void attn_decode_kernel(AttnParams 
         *reinterpret_cast<f32x4_t*>(p.ws_o + prow * 128 + d4) = acc;
         if ((tid & 31) == 0) p.ws_lse[prow] = lse2;
     }
+}
+
+// The pages of the item's first block that another request reads too (requests that share a prefix
+// share its leading blocks at the same places; entries past a request's last block are not read).
+__device__ __forceinline__ bool shares_pages(const AttnParams& p, const Item& it) {
+    const int hk = it.row - it.b * p.s.Hkv;
+    const int e0 = it.split * ((p.nkb[it.b] + p.sp[it.b] - 1) / p.sp[it.b]);
+    if (e0 >= p.nkb[it.b]) return false;
+    const int o = threadIdx.x & 63;  // another request (there are at most 64)
+    const bool other = o < p.s.B && o != it.b && p.nkb[o] > e0;
+    const int64_t at = (int64_t)((other ? o : it.b) * p.s.Hkv + hk) * p.k.pts + e0;
+    const int id = p.k.page_table[at];
+    return __ballot(other && id == sload(p.k.page_table + (int64_t)it.row * p.k.pts + e0)) != 0;
+}
+
+// How K and V are loaded (launch_attn): to stay in the caches, past them, or past them where no other
+// request reads the item's pages.
+enum { kLoadsKept, kLoadsStreamed, kLoadsStreamedUnshared };
+template <int kLoads>
+__global__ __launch_bounds__(kDecWaves * 64) void attn_decode_kernel(AttnParams p) {
+    __shared__ __attribute__((aligned(16))) uint8_t smem[kDecWaves * kDecVBytes];
+    Item it;
+    if (!find_item(p, 1, &it)) return;
+    it.row = __builtin_amdgcn_readfirstlane(it.row);
+    it.b = __builtin_amdgcn_readfirstlane(it.b);
+    it.split = __builtin_amdgcn_readfirstlane(it.split);
+    if (kLoads == kLoadsStreamed || (kLoads == kLoadsStreamedUnshared && !shares_pages(p, it)))
+        decode_item<true>(p, it, smem);
+    else
+        decode_item<false>(p, it, smem);
 }
 
 }  // namespace
@@ -1384,20 +1410,29 @@ hipError_t launch_attn(const AttnArgs& a, hipStream_t stream) {
                     a.v.sblk == 64 * a.v.stok && (int64_t)max_tokens * stok * 2 + 64 * stok * 2 < (int64_t{1} << 31);
     }
     auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(p.per_xcd * 8), dim3(kNW * 64), 0, stream, p); };
-    // A decode launch reads its K and V once.  When they are a good deal more than the last-level
-    // cache (256 MB) holds, nothing useful of them is left there for a next launch, and loads that
-    // do not allocate in it are faster: 8 heads x 131072 tokens (537 MB) 100.4 us, 89.6 us
-    // non-temporal; 81920 tokens (336 MB) 64.0, 60.4.  Nearer to its size a cache read again at
-    // once is partly found there: 73728 tokens 54.7, 55.2; 49152 38.8, 41.2; four 4096-token
-    // requests (67 MB) 18.9, 19.4 (several caches in turn: 73728 tokens 61.0, 55.8; 49152 45.3, 42.2).
+    // A decode launch of requests that share nothing reads its K and V once.  When they are a good deal
+    // more than the last-level cache (256 MB) holds, nothing useful of them is left there for a next
+    // launch, and loads that do not allocate in it are faster: 8 heads x 131072 tokens (537 MB)
+    // 100.4 us, 89.6 us non-temporal; 81920 tokens (336 MB) 64.0, 60.4.  Nearer to its size a cache
+    // read again at once is partly found there: 73728 tokens 54.7, 55.2; 49152 38.8, 41.2; four
+    // 4096-token requests (67 MB) 18.9, 19.4.  Several caches in turn, a model's layers, gain from
+    // less on (73728 tokens 61.0, 55.8; 49152 45.3, 42.2): for them the line lies too high.
+    // What several requests read is kept: the kernel looks for shared pages, stride 0 shows here.  Two
+    // requests on the same pages of 131072 tokens 123 us kept, 147 non-temporal; eight 344, 511.
     constexpr int64_t kStreamBytes = int64_t{320} << 20;
     int64_t kv_bytes = 0;
     for (int b = 0; a.kv_len != nullptr && b < a.s.B; ++b) kv_bytes += (int64_t)a.kv_len[b] * a.s.Hkv * (2 * kD * 2);
+    auto repeats = [&](const KvAddr& t) {
+        return t.page_table == nullptr && ((a.s.B > 1 && t.sb == 0) || (a.s.Hkv > 1 && t.sh == 0));
+    };
+    const bool streamed = kv_bytes >= kStreamBytes && !repeats(a.k) && !repeats(a.v);
     static_assert(kNW == kDecWaves, "one workgroup size for the attention kernels");
     if (a.table)
         row_res ? launch(attn_fwd_kernel<kNW, true, true>) : launch(attn_fwd_kernel<kNW, true, false>);
     else if (attn_uses_decode_kernel(a.s, true))
-        kv_bytes >= kStreamBytes ? launch(attn_decode_kernel<true>) : launch(attn_decode_kernel<false>);
+        !streamed                                    ? launch(attn_decode_kernel<kLoadsKept>)
+        : a.k.page_table != nullptr && a.s.B > 1 ? launch(attn_decode_kernel<kLoadsStreamedUnshared>)
+                                                     : launch(attn_decode_kernel<kLoadsStreamed>);
     else
         row_res ? launch(attn_fwd_kernel<kNW, false, true>) : launch(attn_fwd_kernel<kNW, false, false>);
     hipError_t e = hipGetLastError();
