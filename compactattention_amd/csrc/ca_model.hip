@@ -98,17 +98,18 @@ struct RmsParams {
 
 constexpr int kRmsKeep = 4;  // chunks per thread held in registers: rows up to 8192 elements
 
-// Bound by memory.  kStream: rows held in registers are loaded and stored non-temporally, so they
-// stay out of the way of the product that reads the output next (when: launch_rmsnorm).
-template <bool kStream>
+// Bound by memory.  kStream (when: launch_rmsnorm): a row held in registers is stored
+// non-temporally (kStreamOut), or loaded so too (kStreamAll).
+enum { kStreamNone, kStreamOut, kStreamAll };
+template <int kStream>
 __global__ __launch_bounds__(256) void rmsnorm_kernel(RmsParams p) {
     auto get = [](const uint16_t* a) {
         const u16x8_t* v = reinterpret_cast<const u16x8_t*>(a);
-        return kStream ? __builtin_nontemporal_load(v) : *v;
+        return kStream == kStreamAll ? __builtin_nontemporal_load(v) : *v;
     };
     auto put = [](uint16_t* a, u16x8_t x) {
         u16x8_t* v = reinterpret_cast<u16x8_t*>(a);
-        if (kStream)
+        if (kStream != kStreamNone)
             __builtin_nontemporal_store(x, v);
         else
             *v = x;
@@ -235,16 +236,28 @@ hipError_t launch_rmsnorm(const uint16_t* x, int64_t x_stride, const uint16_t* r
     p.y_stride = y_stride;
     p.n = n;
     p.eps = eps;
-    // Non-temporal up to 16 MB per tensor (half of the eight 4 MB L2s) and while a row fits the
-    // registers, with the residual: 2048 rows of 4096 14.9 -> 13.1 us, 512 of 4096 6.1 -> 5.5,
-    // 2048 of 2048 8.4 -> 7.9; 512 rows of 4096 in a norm -> product -> SwiGLU -> product chain
-    // 206 -> 203 us.  Beyond, caches that keep the rows are faster: 8192 rows of 4096 43.1 us, 47.0
-    // non-temporal, 2048 of 8192 25.9 and 26.7; longer rows are read again: 512 of 16384 18.3 and 21.8.
-    const bool stream_rows = n <= 2048 * kRmsKeep && rows * n <= int64_t{8} << 20;
+    // Non-temporal stores from 4 to 16 MB per tensor, in rows of 2048 elements to what the registers hold
+    // (longer rows are read again).  Times with the residual, kept and so stored, alone on eight sets of
+    // buffers in turn / between two products: 512 rows of 4096 7.2, 6.6 / 40.3, 39.7 us; 1024 9.4, 8.5 /
+    // 47.6, 47.7; 512 of 8192 10.9, 10.0 / 61.5, 61.3.  Below 4 MB, and with shorter rows, the product that
+    // reads the output loses more (256 of 2048 25.1, 25.9; 1024 of 1024 27.1, 29.0; 3072 of 1024 without the
+    // residual 34.6, 35.1), and beyond 16 MB the norm itself (3072 of 4096 22.0, 23.3).
+    // Loads too from 12 MB on: the norm alone loses again (2048 of 4096 15.8 kept, 14.1 stores, 15.4
+    // both), but what streams after it gains more: with the rotation and the SwiGLU product of its
+    // layer 64.8, 64.0, 61.7; 1700 rows 56.5, 55.4, 54.6.  In smaller launches they cost the norm what the
+    // stores give it (1024 of 4096 9.4, 8.5, 9.4; 512 of 8192 10.9, 10.0, 11.5) and the layer nothing.
+    int stream_rows = kStreamNone;
+    if (n >= 2048 && n <= 2048 * kRmsKeep && rows * n >= int64_t{2} << 20 && rows * n <= int64_t{8} << 20)
+        stream_rows = rows * n <= int64_t{6} << 20 ? kStreamOut : kStreamAll;
     auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(rows)), dim3(256), 0, stream, p);
     };
-    stream_rows ? launch(rmsnorm_kernel<true>) : launch(rmsnorm_kernel<false>);
+    if (stream_rows == kStreamAll)
+        launch(rmsnorm_kernel<kStreamAll>);
+    else if (stream_rows == kStreamOut)
+        launch(rmsnorm_kernel<kStreamOut>);
+    else
+        launch(rmsnorm_kernel<kStreamNone>);
     return hipGetLastError();
 }
 

@@ -81,3 +81,18 @@ def test_rmsnorm_same_rows_in_launches_of_any_size(gpu, n, residual):
     whole = norm(x, r)
     for part in (slice(0, rows - 1), slice(rows - 1, rows), slice(3, 70)):
         assert torch.equal(whole[..., part, :], norm(x[part], r[part]))
+
+
+@pytest.mark.parametrize("n", [1024, 2040, 2048, 4096])
+@pytest.mark.parametrize("elements", [2 << 20, 6 << 20])
+def test_rmsnorm_around_its_streamed_sizes(gpu, n, elements):
+    """Launches of one row less than a size from which rows are streamed, of that size and one row more."""
+    print(f"case: rmsnorm n={n} elements={elements}", flush=True)
+    rows = -(-elements // n)
+    g = torch.Generator(device=gpu).manual_seed(n)
+    x, r = (torch.randn((rows + 1, n), generator=g, device=gpu).to(torch.bfloat16) for _ in range(2))
+    w = torch.randn((n,), generator=g, device=gpu).to(torch.bfloat16)
+    few = torch.cat([torch.stack(ops.rmsnorm(x[i:i + 400], w, 1e-5, residual=r[i:i + 400]))
+                     for i in range(0, rows + 1, 400)], 1)
+    for m in (rows - 1, rows, rows + 1):
+        assert torch.equal(torch.stack(ops.rmsnorm(x[:m], w, 1e-5, residual=r[:m])), few[:, :m])
