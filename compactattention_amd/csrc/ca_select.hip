@@ -490,8 +490,8 @@ __device__ __forceinline__ int wave_kth_smallest_id(const int (&id)[S], const bo
     return T;
 }
 
-// A lower bound of the k-th largest of the wave's 64 values (k >= 1): their k-th largest upper
-// half, in 16 rounds.  Half the rounds of the exact one, for a few more candidates above it.
+// The k-th largest of the wave's 64 values (k >= 1) in two steps of 16 rounds: its upper half, a lower
+// bound that lets a few more candidates pass (many where the row's keys are nearly equal), and the rest.
 __device__ __forceinline__ uint32_t wave_kth_bound(uint32_t x, int k) {
     const uint32_t hi = x >> 16;
     uint32_t T = 0;
@@ -501,6 +501,13 @@ __device__ __forceinline__ uint32_t wave_kth_bound(uint32_t x, int k) {
         if (__popcll(__ballot(hi >= c)) >= k) T = c;
     }
     return T << 16;
+}
+__device__ __forceinline__ uint32_t wave_kth_from_bound(uint32_t x, int k, uint32_t T) {
+    for (int bit = 15; bit >= 0; --bit) {
+        const uint32_t c = T | (1u << bit);
+        if (__popcll(__ballot(x >= c)) >= k) T = c;
+    }
+    return T;
 }
 
 // select_candidates for nl <= 64 candidates, one per lane: each counts the candidates before it in
@@ -706,7 +713,9 @@ __global__ __launch_bounds__(kSelThreads) void row_select_kernel(SelectParams p)
         if (wave == 0) {
             uint32_t lo = 0;
             if (k <= 64) {
-                lo = wave_kth_bound(max(max(tmax[lane], tmax[lane + 64]), max(tmax[lane + 128], tmax[lane + 192])), k);
+                const uint32_t m[1] = {max(max(tmax[lane], tmax[lane + 64]),
+                                           max(tmax[lane + 128], tmax[lane + 192]))};
+                lo = wave_kth_largest<1>(m, k);
             }
             if (lane == 0) sel_lo = lo;
         }
@@ -834,10 +843,13 @@ __device__ __forceinline__ float div_by(float v, float sum, float y) {
 //    serves the bound, the candidate list and the masks;
 //  - each wave lists its candidates by ballots in its own part of the list, and every wave
 //    derives the top-k bound and the final cut itself;
-//  - a candidate list that overflows falls back to the whole-row search.
+//  - a candidate list that is long for keys that differ in their lower halves only is made again from
+//    the exact bound; one that overflows all the same falls back to the whole-row search.
 // Results are bit-identical to row_select_kernel.  Bound by the latency of its phases, which is
 // what these choices cut: 512 rows of 2064 blocks, top-k 10, 16.2 -> 12.7 us; 896 rows of up to
-// 2056 17.0 -> 12.7; 256 rows of 1032 9.4 -> 7.1; 128 rows of 128 6.2 -> 4.9.
+// 2056 17.0 -> 12.7; 256 rows of 1032 9.4 -> 7.1; 128 rows of 128 6.2 -> 4.9.  Logits and selection of
+// 512 rows of 2064 blocks, top-k 10: 19.7 us; of nearly equal scores 21.2 (25.1 before the loose bound, 159
+// without the exact one).
 template <bool kCompute, int NR>
 __global__ __launch_bounds__(kSelThreads) void row_select_reg_kernel(SelectParams p) {
     extern __shared__ float row[];  // [cap]
@@ -845,7 +857,7 @@ __global__ __launch_bounds__(kSelThreads) void row_select_reg_kernel(SelectParam
     __shared__ float red_m[kSelWaves];  // its own slots: the statistics reuse no array without a barrier
     __shared__ int red_i[kSelWaves];
     __shared__ int red_z[kSelWaves];
-    __shared__ int red_n[kSelWaves];
+    __shared__ int red_n[2][kSelWaves];
     __shared__ uint32_t tmax[kSelThreads];
     __shared__ uint32_t cand_key[kSelWaves][kCandCap];
     __shared__ int cand_id[kSelWaves][kCandCap];
@@ -995,28 +1007,34 @@ __global__ __launch_bounds__(kSelThreads) void row_select_reg_kernel(SelectParam
         take_all = k >= red_i[0] + red_i[1] + red_i[2] + red_i[3];
         if (!take_all) {
             // every wave computes the same lower bound from the 64 lane maxima (1: any candidate)
-            uint32_t lo = 1;
-            if (k <= 64)
-                lo = max(1u, wave_kth_bound(
-                                 max(max(tmax[lane], tmax[lane + 64]), max(tmax[lane + 128], tmax[lane + 192])), k));
-            int mine = 0;
+            const uint32_t top = max(max(tmax[lane], tmax[lane + 64]), max(tmax[lane + 128], tmax[lane + 192]));
             const uint64_t lt_mask = (1ull << lane) - 1ull;
+            int n0, n1, n2, nl;
+            auto list = [&](uint32_t lo, int (&len)[kSelWaves]) {
+                int mine = 0;
 #pragma unroll
-            for (int i = 0; i < NR; ++i) {
-                const bool c = key[i] >= lo;
-                const uint64_t bal = __ballot(c);
-                if (bal != 0) {
-                    const int slot = mine + __popcll(bal & lt_mask);
-                    if (c && slot < kCandCap) {
-                        cand_key[wave][slot] = key[i];
-                        cand_id[wave][slot] = t + kSelThreads * i;
+                for (int i = 0; i < NR; ++i) {
+                    const bool c = key[i] >= lo;
+                    const uint64_t bal = __ballot(c);
+                    if (bal != 0) {
+                        const int slot = mine + __popcll(bal & lt_mask);
+                        if (c && slot < kCandCap) {
+                            cand_key[wave][slot] = key[i];
+                            cand_id[wave][slot] = t + kSelThreads * i;
+                        }
+                        mine += __popcll(bal);
                     }
-                    mine += __popcll(bal);
                 }
+                if (lane == 0) len[wave] = mine;
+                __syncthreads();
+                n0 = len[0], n1 = n0 + len[1], n2 = n1 + len[2], nl = n2 + len[3];
+            };
+            const uint32_t bound = k <= 64 ? wave_kth_bound(top, k) : 0u;
+            list(max(1u, bound), red_n[0]);
+            if (k <= 64 && nl > (k <= 32 ? 64 : kCandCap)) {
+                const uint32_t lo = wave_kth_from_bound(top, k, bound);
+                if (lo != bound) list(lo, red_n[1]);
             }
-            if (lane == 0) red_n[wave] = mine;
-            __syncthreads();
-            const int n0 = red_n[0], n1 = n0 + red_n[1], n2 = n1 + red_n[2], nl = n2 + red_n[3];
             auto cand = [&](int j, uint32_t& ck, int& ci) {  // entry j of the four waves' lists in a row
                 const int wv = (j >= n0) + (j >= n1) + (j >= n2);
                 const int at = j - (wv == 0 ? 0 : wv == 1 ? n0 : wv == 2 ? n1 : n2);

@@ -46,3 +46,25 @@ def test_row_lengths(gpu, cap):
 @pytest.mark.parametrize("past", [100, 1500])
 def test_peaked_rows(gpu, past, spread):
     _check(gpu, [past], 1, 4, 3, spread, seed=past)
+
+
+@pytest.mark.parametrize("cap", [70, 257, 600, 1500, 2304, 4000, 4200])
+def test_nearly_equal_scores_and_many_picks(gpu, cap):
+    """Rows whose keys agree in their upper halves, tie, or hold what is no candidate, and more picks than
+    a candidate list holds."""
+    print(f"case: nearly equal scores cap={cap}", flush=True)
+    past, Hkv, G, Qb = [cap - 2, (cap - 2) // 2], 1, 2, 2
+    g = torch.Generator().manual_seed(cap)
+    x = torch.rand((2, Hkv * G, Qb, cap), generator=g)
+    odd = x.clone()
+    odd[..., ::7] = float("nan")
+    odd[..., 3::11] = float("-inf")
+    rows = {"near": 1 + 1e-3 * x, "nearer": 1 + 2e-6 * x, "negative": -1 - 1e-3 * x, "equal": torch.ones_like(x),
+            "few": (x * 3).floor(), "late": torch.where(x < 0.9, 0.0, 1 + 1e-4 * x), "odd": 1 + 1e-3 * odd}
+    for name, s in rows.items():
+        for k in (1, 10, 32, 33, 64, 65, 300):
+            for cols in (False, True):
+                rule = dict(topk=k, topk_all_columns=cols)
+                got = ops.select_scores(s.to(gpu), ops.Rule(**rule), past, Hkv, cap, 64 * Qb)
+                want = oracle.select_rows(s.numpy(), past, oracle.Rule(**rule))
+                assert np.array_equal(unpack_rowmask(got, cap), want), (name, k, cols)
