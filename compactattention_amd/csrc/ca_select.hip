@@ -547,6 +547,26 @@ __device__ __forceinline__ void select_candidates(const uint32_t (&x)[S], const 
     eq_cut = wave_kth_smallest_id<S>(id, eq, k - gt);
 }
 
+// The k-th largest key T >= 1 of the row by all waves of the workgroup, 32 rounds of a count and a
+// barrier, and the number of keys above it.  count(c): the wave's keys >= c.
+template <typename Count>
+__device__ __forceinline__ uint32_t row_kth_largest(int (&red)[2][kSelWaves], int k, int wave, int lane, int* above,
+                                                    Count count) {
+    auto total = [&](int slot, uint32_t c) {  // (a slot is written again two barriers later)
+        const int mine = count(c);
+        if (lane == 0) red[slot][wave] = mine;
+        __syncthreads();
+        return red[slot][0] + red[slot][1] + red[slot][2] + red[slot][3];
+    };
+    uint32_t T = 0;
+    for (int bit = 31; bit >= 0; --bit) {
+        const uint32_t c = T | (1u << bit);
+        if (total(bit & 1, c) >= k) T = c;
+    }
+    *above = total(1, T + 1);
+    return T;
+}
+
 template <bool kCompute>
 __global__ __launch_bounds__(kSelThreads) void row_select_kernel(SelectParams p) {
     extern __shared__ float row[];  // [cap]
@@ -559,6 +579,7 @@ __global__ __launch_bounds__(kSelThreads) void row_select_kernel(SelectParams p)
     __shared__ int cand_n;
     __shared__ uint32_t sel_lo, sel_T;
     __shared__ int sel_cut;
+    __shared__ int red_k[2][kSelWaves];
     const Shape& s = p.s;
     const int rid = blockIdx.x;  // (b*Hq + h)*Qb + qb
     const int qb = rid % s.Qb;
@@ -733,9 +754,19 @@ __global__ __launch_bounds__(kSelThreads) void row_select_kernel(SelectParams p)
             }
         }
         __syncthreads();
+        const int nl = cand_n;
+        uint32_t T = 0;
+        int above = 0;
+        if (nl > kCandCap)  // heavy ties or k > 64
+            T = row_kth_largest(red_k, k, wave, lane, &above, [&](uint32_t c) {
+                int cnt = 0;
+                for (int kb = t; kb < kend; kb += kSelThreads) {
+                    float v;
+                    cnt += (cand_val(kb, v) && order_key(v) >= c) ? 1 : 0;
+                }
+                return wave_sum_int(cnt);
+            });
         if (wave == 0) {
-            const int nl = cand_n;
-            uint32_t T;
             int eq_cut;
             if (nl <= 64) {
                 // the usual case: one candidate per lane
@@ -751,22 +782,7 @@ __global__ __launch_bounds__(kSelThreads) void row_select_kernel(SelectParams p)
                 }
                 select_candidates<kCandSlots>(x, id, k, T, eq_cut);
             } else {
-                T = 0;
-                for (int bit = 31; bit >= 0; --bit) {
-                    const uint32_t c = T | (1u << bit);
-                    int cnt = 0;
-                    for (int kb = lane; kb < kend; kb += 64) {
-                        float v;
-                        cnt += (cand_val(kb, v) && order_key(v) >= c) ? 1 : 0;
-                    }
-                    if (wave_sum_int(cnt) >= k) T = c;
-                }
-                int gt = 0;
-                for (int kb = lane; kb < kend; kb += 64) {
-                    float v;
-                    gt += (cand_val(kb, v) && order_key(v) > T) ? 1 : 0;
-                }
-                const int krem = k - wave_sum_int(gt);
+                const int krem = k - above;
                 // the krem-th key equal to T in ascending block order
                 const uint64_t lt_mask = (1ull << lane) - 1ull;
                 int seen = 0;
@@ -844,15 +860,15 @@ __device__ __forceinline__ float div_by(float v, float sum, float y) {
 //  - each wave lists its candidates by ballots in its own part of the list, and every wave
 //    derives the top-k bound and the final cut itself;
 //  - a candidate list that is long for keys that differ in their lower halves only is made again from
-//    the exact bound; one that overflows all the same falls back to the whole-row search.
+//    the exact bound; one that overflows all the same falls back to a search of all keys.
 // Results are bit-identical to row_select_kernel.  Bound by the latency of its phases, which is
 // what these choices cut: 512 rows of 2064 blocks, top-k 10, 16.2 -> 12.7 us; 896 rows of up to
 // 2056 17.0 -> 12.7; 256 rows of 1032 9.4 -> 7.1; 128 rows of 128 6.2 -> 4.9.  Logits and selection of
-// 512 rows of 2064 blocks, top-k 10: 19.7 us; of nearly equal scores 21.2 (25.1 before the loose bound, 159
-// without the exact one).
+// 512 rows of 2064 blocks: top-k 10 19.7 us; top-k 200 26.6 (150 with the search by one wave in LDS);
+// top-k 10 of nearly equal scores 21.2 (25.1 before the loose bound, 159 without the exact one).
 template <bool kCompute, int NR>
 __global__ __launch_bounds__(kSelThreads) void row_select_reg_kernel(SelectParams p) {
-    extern __shared__ float row[];  // [cap]
+    extern __shared__ float row[];  // [cap]: the exponentials of the softmax
     __shared__ float red_f[kSelWaves];
     __shared__ float red_m[kSelWaves];  // its own slots: the statistics reuse no array without a barrier
     __shared__ int red_i[kSelWaves];
@@ -861,8 +877,8 @@ __global__ __launch_bounds__(kSelThreads) void row_select_reg_kernel(SelectParam
     __shared__ uint32_t tmax[kSelThreads];
     __shared__ uint32_t cand_key[kSelWaves][kCandCap];
     __shared__ int cand_id[kSelWaves][kCandCap];
-    __shared__ uint32_t sel_T;
-    __shared__ int sel_cut;
+    __shared__ int red_k[2][kSelWaves];
+    __shared__ uint64_t eq_bits[kSelWaves * NR];
     const Shape& s = p.s;
     const int rid = blockIdx.x;  // (b*Hq + h)*Qb + qb
     const int qb = rid % s.Qb;
@@ -1053,61 +1069,33 @@ __global__ __launch_bounds__(kSelThreads) void row_select_reg_kernel(SelectParam
                 for (int i = 0; i < kCandSlots; ++i) cand(lane + 64 * i, ck[i], ci[i]);
                 select_candidates<kCandSlots>(ck, ci, k, T, eq_cut);
             } else {
-                // heavy ties or k > 64: the row goes to LDS and wave 0 searches it, as
-                // row_select_kernel does (the exponentials there were last read before the barriers above)
+                // heavy ties or k > 64: the row's keys are searched where they are
+                int above;
+                T = row_kth_largest(red_k, k, wave, lane, &above, [&](uint32_t c) {
+                    int cnt = 0;
 #pragma unroll
-                for (int i = 0; i < NR; ++i)
-                    if (t + kSelThreads * i < n) row[t + kSelThreads * i] = v[i];
-                __syncthreads();
-                if (wave == 0) {
-                    auto row_val = [&](int kb, float& cv) -> bool {
-                        if (all_cols) {
-                            cv = kb < n ? row[kb] : 0.0f;
-                            if (!is_finite_f(cv)) cv = 0.0f;
-                            return true;
-                        }
-                        cv = row[kb];
-                        return is_finite_f(cv);
-                    };
-                    uint32_t Tw = 0;
-                    for (int bit = 31; bit >= 0; --bit) {
-                        const uint32_t c = Tw | (1u << bit);
-                        int cnt = 0;
-                        for (int kb = lane; kb < kend; kb += 64) {
-                            float cv;
-                            cnt += (row_val(kb, cv) && order_key(cv) >= c) ? 1 : 0;
-                        }
-                        if (wave_sum_int(cnt) >= k) Tw = c;
-                    }
-                    int gt = 0;
-                    for (int kb = lane; kb < kend; kb += 64) {
-                        float cv;
-                        gt += (row_val(kb, cv) && order_key(cv) > Tw) ? 1 : 0;
-                    }
-                    const int krem = k - wave_sum_int(gt);
-                    int seen = 0;
-                    int cutw = kend;
-                    for (int base = 0; base < kend; base += 64) {
-                        const int kb = base + lane;
-                        float cv = 0.0f;
-                        const bool e = kb < kend && row_val(kb, cv) && order_key(cv) == Tw;
-                        const uint64_t bal = __ballot(e);
-                        const int cnt = __popcll(bal);
-                        if (seen + cnt >= krem) {
-                            const uint64_t who = __ballot(e && seen + __popcll(bal & lt_mask) == krem - 1);
-                            cutw = base + __ffsll(static_cast<unsigned long long>(who)) - 1;
-                            break;
-                        }
-                        seen += cnt;
-                    }
-                    if (lane == 0) {
-                        sel_T = Tw;
-                        sel_cut = cutw;
-                    }
+                    for (int i = 0; i < NR; ++i) cnt += __popcll(__ballot(key[i] >= c));
+                    return cnt;
+                });
+                // the (k - above)-th key equal to T in ascending block order: the chunk that holds it, then its bit
+#pragma unroll
+                for (int i = 0; i < NR; ++i) {
+                    const uint64_t bal = __ballot(key[i] == T);
+                    if (lane == 0) eq_bits[wave + kSelWaves * i] = bal;
                 }
                 __syncthreads();
-                T = sel_T;
-                eq_cut = sel_cut;
+                const uint64_t bits = lane < kSelWaves * NR ? eq_bits[lane] : 0;
+                int upto = __popcll(bits);
+#pragma unroll
+                for (int o = 1; o < 64; o <<= 1) {
+                    const int y = __shfl_up(upto, o, 64);
+                    if (lane >= o) upto += y;
+                }
+                const int c = __ffsll(static_cast<unsigned long long>(__ballot(upto >= k - above))) - 1;
+                const uint64_t chunk = eq_bits[c];
+                const int nth = k - above - (__builtin_amdgcn_readlane(upto, c) - __popcll(chunk));
+                const uint64_t who = __ballot((chunk >> lane & 1) && __popcll(chunk & lt_mask) == nth - 1);
+                eq_cut = 64 * c + __ffsll(static_cast<unsigned long long>(who)) - 1;
             }
         }
     }
