@@ -438,6 +438,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
     // and 0 * V must not meet a non-finite V).  Row offsets go in the VGPR offset, which the
     // range check covers.
     const int kv_tokens = qpos0 + s.Lq;
+    const int last_rows = kv_tokens - 64 * (nkb - 1);  // of the last block
     const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(to_lds(smem))) + wu * 1024;
     // Where a block's rows are: its logical id (kRow: the offset in the row's one resource) and
     // its K and V pages.  The id nkb, the block after the request's last, stands for no block:
@@ -456,7 +457,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
             // scalar offset is not checked)
             off += id * 64 * stok_b;
         else
-            rsrc = buffer_words(base_row + page * sblk, max(min(kv_tokens - id * 64, 64), 0) * stok_b);
+            rsrc = buffer_words(base_row + page * sblk, id < nkb - 1 ? 64 * stok_b : id < nkb ? last_rows * stok_b : 0);
         dma_lds<kRow>(rsrc, off, dst + half * 8192);
     };
     // The list's blocks, 64 entries at a time in registers (lane i: entry 64 c + i, no block past
@@ -534,9 +535,19 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
         for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
             for (int j = 0; j < 16; ++j) sc[kt][j] = 0.0f;
+        bf16x8_t kr[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) kr[i] = k_frag(kbase, i);
 #pragma unroll
         for (int i = 0; i < 16; ++i)
-            sc[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k_frag(kbase, i), qf[i >> 1], sc[i & 1], 0, 0, 0);
+            sc[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kr[i], qf[i >> 1], sc[i & 1], 0, 0, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);  // 6 LDS reads
+#pragma unroll
+        for (int i = 0; i < 10; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // 1 MFMA
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // 1 LDS read
+        }
+        __builtin_amdgcn_sched_group_barrier(0x008, 6, 0);
     };
     auto mask = [&](int kb) {
         // value j of half kt holds key kt*32 + swap23(8*(j/4) + 4*h + j%4)
@@ -601,8 +612,9 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
     // slot j stands for: K of block j + 2 and V of block j + 1 have landed, and every wave has
     // read K of block j + 1 and V of block j - 1.  So slot j issues V of block j + 3 and K of
     // block j + 5 after it, into the places of those two in rings of four blocks, and the
-    // loads stay in flight for two (V) and three (K) slots.  Every slot issues its four loads
-    // (blocks past the list's end load nothing), so the counts of the waits are constants.
+    // loads stay in flight for two (V) and three (K) slots.  A pipelined slot issues its four loads
+    // always (blocks past the list's end load nothing), so the count of its wait is a constant; the
+    // prologue and the other slots leave out what the list does not have, and then wait for all.
     Blk vq0, vq1;  // the two entries whose K is issued and V is not
     auto issue_k = [&](int i, int half, const Blk& b) {
         load_half(kbase_row, k_rsrc, p.k.sblk, kstok_b, k_goff, b.id, b.kp, half, lds0 + (i & 3) * 16384);
@@ -610,13 +622,17 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
     auto issue_v = [&](int i, int half, const Blk& b) {
         load_half(vbase_row, v_rsrc, p.v.sblk, vstok_b, v_goff, b.id, b.vp, half, lds0 + kVRing + (i & 3) * 16384);
     };
-    auto mid_slot = [&]() {
+    auto mid_slot = [&](bool all) {
         // K of j + 3, V of j + 2 and K of j + 4 may stay in flight
-        asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+        if (all)
+            wait_dma();
+        else
+            asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         CA_PIN();
     };
     auto issue_slot = [&](int j) {
+        if (j + 3 >= nblk) return;
         const Blk nb = next_blk(j + 5);
         for (int half = 0; half < 2; ++half) issue_v(j + 3, half, vq0);
         for (int half = 0; half < 2; ++half) issue_k(j + 5, half, nb);
@@ -666,7 +682,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
             asm volatile("" : "+v"(sn[i & 1]), "+v"(y[e - 1]), "+v"(x[e - 2]), "+v"(rs), "+v"(sc[e >> 4]) : : "memory");
             __builtin_amdgcn_sched_barrier(0);
         }
-        mid_slot();
+        mid_slot(false);
         // a wave in its PV half, whose groups are shorter, goes before one in its scores (-0.5 %)
         __builtin_amdgcn_s_setprio(1);
         const Blk nb = next_blk(j + 5);
@@ -709,18 +725,26 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
         const Blk b0 = next_blk(0), b1 = next_blk(1);
         vq0 = next_blk(2);
         vq1 = next_blk(3);
+        const bool few = nblk < 4;
         for (int half = 0; half < 2; ++half) issue_k(0, half, b0);
-        for (int half = 0; half < 2; ++half) issue_k(1, half, b1);
+        if (nblk > 1)
+            for (int half = 0; half < 2; ++half) issue_k(1, half, b1);
         for (int half = 0; half < 2; ++half) issue_v(0, half, b0);
-        for (int half = 0; half < 2; ++half) issue_k(2, half, vq0);
-        for (int half = 0; half < 2; ++half) issue_v(1, half, b1);
-        for (int half = 0; half < 2; ++half) issue_k(3, half, vq1);
-        asm volatile("s_waitcnt vmcnt(10)" ::: "memory");
+        if (nblk > 2)
+            for (int half = 0; half < 2; ++half) issue_k(2, half, vq0);
+        if (nblk > 1)
+            for (int half = 0; half < 2; ++half) issue_v(1, half, b1);
+        if (!few)
+            for (int half = 0; half < 2; ++half) issue_k(3, half, vq1);
+        if (few)
+            wait_dma();
+        else
+            asm volatile("s_waitcnt vmcnt(10)" ::: "memory");
         __syncthreads();
         scores(0);
         if (n_un == 0) mask(block_id(e0));
         block_max();
-        mid_slot();
+        mid_slot(few);
         issue_slot(-1);
         int j = 0;
         f32x16_t sn[2];
@@ -745,7 +769,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
                 scores(((j + 1) & 3) * 16384);
                 if (j + 1 >= n_un) mask(block_id(e0 + j + 1));
                 block_max();
-                mid_slot();
+                mid_slot(j + 2 >= nblk);
                 issue_slot(j);
             }
         }
