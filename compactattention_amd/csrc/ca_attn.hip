@@ -373,7 +373,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
         n_vis = -1;
         for (;; end -= 64) {
             const int e = end - 1 - l;
-            const int id = e >= 0 ? tab[e] : -1;
+            const int id = e >= 0 ? max(tab[e], 0) : -1;
             if (n_vis < 0) {
                 const uint64_t seen = __ballot(id <= lim);
                 if (seen == 0) continue;

@@ -163,3 +163,22 @@ def test_ragged_decode_placement(gpu, lens, splits):
             err = (out[b, 0, 2 * h:2 * h + 2].float() - torch.softmax(s, -1) @ v[b, h, :n].float()).abs()
             # the attention tolerances: weights are rounded to bf16, an output is a mean under them
             assert err.max() <= 2e-2 and err.mean() <= 2e-3, (b, h, err.max(), err.mean())
+
+
+@pytest.mark.parametrize("P", [0, 2])
+def test_ids_outside_the_cache_read_its_ends(gpu, P):
+    """A table's ids are clamped into the request's blocks, for the causal mask as for the reads."""
+    print(f"case: ids outside the cache P={P}", flush=True)
+    Hq, Hkv, Lq = 8, 2, 100
+    cap = P + 2
+    g = torch.Generator().manual_seed(P)
+    q = torch.randn((1, Lq, Hq, 128), generator=g).to(torch.bfloat16).to(gpu)
+    k, v = (torch.randn((1, Hkv, cap * 64, 128), generator=g).to(torch.bfloat16).to(gpu) for _ in range(2))
+    ids = torch.arange(cap, dtype=torch.int32, device=gpu).repeat(Hkv, 1)
+    counts = torch.full((Hkv,), cap, dtype=torch.int32, device=gpu)
+    args = (counts, [P], 1.0 / math.sqrt(128), cap, Hkv)
+    K, V = ops.KV.heads_first(k), ops.KV.heads_first(v)
+    want = ops.attn_fwd(q, K, V, ids, *args)
+    low = ids.clone()
+    low[:, 0] = -5
+    assert torch.equal(ops.attn_fwd(q, K, V, low, *args), want)
