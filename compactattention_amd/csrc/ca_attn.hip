@@ -16,9 +16,9 @@
 //    matrix cores beside the softmax of this one, then its PV product beside the next block's
 //    row max, instruction by instruction (fused below).  Bound: matrix-core issue and power.
 //    At 2048 queries over 32768 dense keys (32 Q / 8 KV heads) a 64-key step of a SIMD's two
-//    waves takes about 3000 cycles for 2176 of MFMA work (72 % busy) where it took 3700 (57 %),
-//    but the part lowers its clock as the matrix cores fill (1.75 -> 1.5 GHz), so the launch
-//    gains 6-7 % (966 -> 906 us); with the loop's LDS reads left out it would gain another 9 %.
+//    waves takes about 3000 cycles for 2176 of MFMA work (73 % busy) where it took 3700 (58 %),
+//    but the part lowers its clock as the matrix cores fill (1.93 -> 1.71 GHz), so the launch
+//    gains 5 % (967 -> 918 us); with the loop's LDS reads left out it would gain another 9 %.
 //  - Scores are computed transposed, S^T = K Q^T (A = K from LDS, B = Q from VGPRs), so the
 //    softmax output lands in exactly the VGPR layout the second product's B operand needs:
 //    O^T += V^T P^T (A = V^T from LDS).  Inside each 32-key S^T tile the A-row -> key map
@@ -28,7 +28,8 @@
 //    row-major with XOR swizzles that keep the fragment reads free of bank conflicts.  V^T
 //    fragments are read with the gfx950 transposing LDS read (ds_read_b64_tr_b16), two
 //    per MFMA.
-//  - Rings of four K and four V blocks in LDS; the DMA runs two (V) and three (K) blocks ahead.
+//  - Rings of four K and four V blocks in LDS.  The slot that finishes block j issues K of j + 5
+//    and V of j + 3, which then stay in flight for three and two slots.
 //    Optional split of each row's block list (split-KV) with an LSE merge.
 //  - Workgroup ids are remapped so consecutive work items (same KV row) share an XCD and
 //    its L2.

@@ -271,9 +271,10 @@ __global__ __launch_bounds__(256) void chunk_summaries_kernel(Shape s, SeqAddr k
 // 4x4x1 form (16 blocks) runs 54 products a cycle and SIMD where four chains alternate, the
 // 16x16x1 one 32 and fmas 16; a step of a wave's 32 x 32 logits reads four floats a lane from
 // LDS.  Few query vectors take a wave of 16 x 64.
-// Bound by latency (launch, loads, 512 MFMAs a wave): kernel times against 4 x 2 register tiles of
-// fmas, 64 vectors x 2064 keys x 8 groups 11.7 -> 11.5 us, 56 x 2056 x 16 ragged 12.0 -> 11.0,
-// 32 x 1032 x 8 8.5 -> 6.9, 16 x 128 x 8 6.4 -> 6.2.
+// Bound by latency (launch, loads, 512 MFMAs a wave): times in a traced chunk step against 4 x 2
+// register tiles of fmas, 56 vectors x 2056 keys x 16 groups ragged 11.7 -> 10.7 us, 32 x 1032 x 8
+// 7.7 -> 6.9, 64 x 2064 x 8 10.7 -> 10.9, 16 x 128 x 8 6.1 -> 6.5 (with the row selection after it
+// 25.2 -> 22.0 and 12.7 -> 11.3).
 constexpr int kPadRow = kD + 4;  // LDS row pitch (floats) for summary tiles
 constexpr int kLogitsKeys = 64;  // key blocks per workgroup
 
@@ -862,8 +863,8 @@ __device__ __forceinline__ float div_by(float v, float sum, float y) {
 //  - a candidate list that is long for keys that differ in their lower halves only is made again from
 //    the exact bound; one that overflows all the same falls back to a search of all keys.
 // Results are bit-identical to row_select_kernel.  Bound by the latency of its phases, which is
-// what these choices cut: 512 rows of 2064 blocks, top-k 10, 16.2 -> 12.7 us; 896 rows of up to
-// 2056 17.0 -> 12.7; 256 rows of 1032 9.4 -> 7.1; 128 rows of 128 6.2 -> 4.9.  Logits and selection of
+// what these choices cut (traced chunk steps): 512 rows of 2064 blocks, top-k 10, 14.5 -> 11.1 us; 896
+// rows of up to 2056 16.5 -> 12.2; 256 rows of 1032 9.2 -> 7.5; 128 rows of 128 6.6 -> 4.9.  Logits and selection of
 // 512 rows of 2064 blocks: top-k 10 19.7 us; top-k 200 26.6 (150 with the search by one wave in LDS);
 // top-k 10 of nearly equal scores 21.2 (25.1 before the loose bound, 159 without the exact one).
 template <bool kCompute, int NR>
